@@ -6,10 +6,12 @@
 // method that the giant steps then rotate and add (exact-residue semantics of
 // bench/cmp/kernels/holmes_mac.cu:8-12, multi-input tiling of holmes_mac.cu:108-190).
 //
-// A thread owns one coefficient of one limb and a TI x TG tile of (input, giant) accumulators for
-// both components: per baby step it reads TG plaintext words and 2 TI baby words for 2 TI TG
-// products (the next step's words are loaded while the current step computes), so plaintexts
-// stream once per input tile and babies once per giant tile.  All tiles
+// A thread owns one coefficient of one limb and
+// a TI x 8 tile of (input, giant) accumulators for both components: per baby step it reads 8 plaintext
+// words and 2 TI baby words for 16 TI products (the next step's words are loaded while the current step
+// computes), so plaintexts stream once per input tile and babies once per giant tile.  Up to 3 inputs HBM
+// bounds it (4.5 to 4.9 TB/s with tiles of just these inputs; a tile of 4 ran 1 input's 512 x 17 limbs in
+// 1.69 ms, where the products of the 3 empty rows bounded it, against 1.19 ms), from 4 on the VALU.  All tiles
 // of one (limb, 128-coefficient) unit are dispatched to the same XCD (workgroups are handed to
 // the 8 XCDs round-robin by linear id), so the unit's plaintext and baby data is fetched from HBM
 // once and then served from that XCD's L2.
@@ -24,16 +26,16 @@ namespace hck {
 namespace {
 
 constexpr int kMacThreads = 128;
-// Register tile: inputs x giants per thread (both components).  Tunable at build time.
-#ifndef HCK_MAC_TI
-#define HCK_MAC_TI 4
-#endif
-#ifndef HCK_MAC_TG
-#define HCK_MAC_TG 8
-#endif
-constexpr int kTI = HCK_MAC_TI;
-constexpr int kTG = HCK_MAC_TG;
+constexpr int kTG = 8;  // giants per thread
 constexpr int kMaxBabies = 64;
+
+// Inputs per thread: the tile that computes the fewest padded rows (measured time per row of the tiles of
+// 4, 3 and 2 inputs 1 : 0.95 : 1.07; a single input has a tile of its own).
+inline int mac_tile_inputs(int ni) {
+  if (ni == 1) return 1;
+  const int c4 = (ni + 3) / 4 * 4 * 100, c3 = (ni + 2) / 3 * 3 * 95, c2 = (ni + 1) / 2 * 2 * 107;
+  return c4 <= c3 && c4 <= c2 ? 4 : c3 <= c2 ? 3 : 2;
+}
 
 struct BabyPtrs {
   const uint64_t* c0[kMaxBabies];
@@ -43,12 +45,14 @@ struct MacPrimes {
   uint8_t prime[kMaxPrimes];
 };
 
-// One baby step's operands for a thread: TG plaintext words, TI words of each component.
+// One baby step's operands for a thread: kTG plaintext words, TI words of each component.
+template <int TI>
 struct MacOps {
-  uint64_t w[kTG], x0[kTI], x1[kTI];
+  uint64_t w[kTG], x0[TI], x1[TI];
 };
 
-__device__ __forceinline__ void mac_load(MacOps& o, const BabyPtrs& babies, int b, int nb, int G, int ni,
+template <int TI>
+__device__ __forceinline__ void mac_load(MacOps<TI>& o, const BabyPtrs& babies, int b, int nb, int G, int ni,
                                          int g0, int i0, const uint64_t* __restrict__ pts, long long pt_stride,
                                          long long baby_stride, long long ln) {
 #pragma unroll
@@ -59,13 +63,14 @@ __device__ __forceinline__ void mac_load(MacOps& o, const BabyPtrs& babies, int 
   const uint64_t* b0 = babies.c0[b];
   const uint64_t* b1 = babies.c1[b];
 #pragma unroll
-  for (int t = 0; t < kTI; ++t) {
+  for (int t = 0; t < TI; ++t) {
     const int ii = i0 + t < ni ? i0 + t : i0;
     o.x0[t] = b0[(long long)ii * baby_stride + ln];
     o.x1[t] = b1[(long long)ii * baby_stride + ln];
   }
 }
 
+template <int TI>
 __global__ __launch_bounds__(kMacThreads) void k_bsgs_mac(uint64_t* __restrict__ res, BabyPtrs babies,
                                                           long long baby_stride, int nb, int ni, int G,
                                                           const uint64_t* __restrict__ pts, long long pt_stride,
@@ -80,19 +85,19 @@ __global__ __launch_bounds__(kMacThreads) void k_bsgs_mac(uint64_t* __restrict__
   if (unit >= total_units) return;
   const int l = unit / units_per_limb;
   const int n = (unit % units_per_limb) * kMacThreads + threadIdx.x;
-  const int i0 = (tile % tiles_i) * kTI, g0 = (tile / tiles_i) * kTG;
+  const int i0 = (tile % tiles_i) * TI, g0 = (tile / tiles_i) * kTG;
   const int pi = mp.prime[l];
   const double p = T.p[pi], pinv = T.pinv[pi];
   const long long ln = (long long)l * kN + n;
-  double acc[kTI][2][kTG];
+  double acc[TI][2][kTG];
 #pragma unroll
-  for (int t = 0; t < kTI; ++t)
+  for (int t = 0; t < TI; ++t)
 #pragma unroll
     for (int c = 0; c < 2; ++c)
 #pragma unroll
       for (int g = 0; g < kTG; ++g) acc[t][c][g] = 0.0;
   // one baby step's products from its loaded words; every 8 steps the sums are reduced
-  auto step = [&](const MacOps& cur, int b) {
+  auto step = [&](const MacOps<TI>& cur, int b) {
     double w[kTG], wp[kTG];
 #pragma unroll
     for (int g = 0; g < kTG; ++g) {
@@ -100,7 +105,7 @@ __global__ __launch_bounds__(kMacThreads) void k_bsgs_mac(uint64_t* __restrict__
       wp[g] = w[g] * pinv;
     }
 #pragma unroll
-    for (int t = 0; t < kTI; ++t) {
+    for (int t = 0; t < TI; ++t) {
       const double x0 = u2d(cur.x0[t]), x1 = u2d(cur.x1[t]);
 #pragma unroll
       for (int g = 0; g < kTG; ++g) {
@@ -110,7 +115,7 @@ __global__ __launch_bounds__(kMacThreads) void k_bsgs_mac(uint64_t* __restrict__
     }
     if ((b & 7) == 7) {
 #pragma unroll
-      for (int t = 0; t < kTI; ++t)
+      for (int t = 0; t < TI; ++t)
 #pragma unroll
         for (int c = 0; c < 2; ++c)
 #pragma unroll
@@ -120,7 +125,7 @@ __global__ __launch_bounds__(kMacThreads) void k_bsgs_mac(uint64_t* __restrict__
   // two-stage software pipeline on two register sets: baby step b + 1's words load into one set while
   // step b computes from the other (the last pair reloads its own words, unused), so the wait before
   // a step's products covers only that step's own loads.
-  MacOps o0, o1;
+  MacOps<TI> o0, o1;
   mac_load(o0, babies, 0, nb, G, ni, g0, i0, pts, pt_stride, baby_stride, ln);
   int b = 0;
   for (; b + 1 < nb; b += 2) {
@@ -138,7 +143,7 @@ __global__ __launch_bounds__(kMacThreads) void k_bsgs_mac(uint64_t* __restrict__
   if (b < nb) step(o0, b);  // odd count: the last step's words are in o0
   const long long is = (long long)limbs * kN, gs = (long long)ni * is, cs = (long long)G * gs;
 #pragma unroll
-  for (int t = 0; t < kTI; ++t) {
+  for (int t = 0; t < TI; ++t) {
     if (i0 + t >= ni) break;
 #pragma unroll
     for (int c = 0; c < 2; ++c)
@@ -271,12 +276,14 @@ extern "C" int hck_bsgs_mac(const hck_context* ctx, int limbs, const int* prime_
   }
   const int units_per_limb = hck::kN / hck::kMacThreads;
   const int total_units = limbs * units_per_limb;
-  const int tiles_i = (inputs + hck::kTI - 1) / hck::kTI, tiles_g = (giants + hck::kTG - 1) / hck::kTG;
+  const int ti = hck::mac_tile_inputs(inputs);
+  const int tiles_i = (inputs + ti - 1) / ti, tiles_g = (giants + hck::kTG - 1) / hck::kTG;
   const int tiles = tiles_i * tiles_g;
   const long long units_padded = ((long long)total_units + hck::kXcds - 1) / hck::kXcds * hck::kXcds;
   const long long blocks = units_padded * tiles;
   if (blocks > 0x7fffffffLL) return HCK_ERR_ARG;
-  hck::k_bsgs_mac<<<dim3((unsigned)blocks), hck::kMacThreads, 0, (hipStream_t)stream>>>(
+  auto k = ti == 1 ? hck::k_bsgs_mac<1> : ti == 2 ? hck::k_bsgs_mac<2> : ti == 3 ? hck::k_bsgs_mac<3> : hck::k_bsgs_mac<4>;
+  k<<<dim3((unsigned)blocks), hck::kMacThreads, 0, (hipStream_t)stream>>>(
       res, bp, baby_stride, babies, inputs, giants, pts, pt_stride, limbs, mp, units_per_limb, tiles_i, tiles_g,
       total_units, ctx->dev);
   HCK_CHECK_LAUNCH();

@@ -1,0 +1,63 @@
+"""GPU parity of the multiply-accumulate's two kernels where their tiles end: the matrix-core kernel's
+16 giants x 16 columns x 16 babies (full, one short, one more, several chunks of babies), the VALU
+kernel's tiles of 1 to 4 inputs x 8 giants, and the rows the vector loads cannot take, bit-exact against
+the oracle on both prime widths."""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+from oracle import oracle as O  # noqa: E402
+
+
+@pytest.fixture(scope="module", params=["50-bit", "59/60-bit"])
+def env(request):
+    from holmes_amd import fhe
+    from holmes_amd.context import CKKSContext
+
+    bits = dict(dcrt_bits=50, first_mod=50) if request.param == "50-bit" else dict(dcrt_bits=59, first_mod=60)
+    ctx = CKKSContext(fhe.CKKSContextSpec(depth=3, dnum=2, seed=5, **bits))
+    return ctx, O.OracleContext(16, ctx.L, ctx.K, ctx.alpha, ctx.primes)
+
+
+def _residues(rng, shape, q):
+    return rng.integers(0, 2**62, size=shape, dtype=np.uint64) % q
+
+
+def _check(env, ni, nb, G, limbs, offset=0):
+    ctx, orc = env
+    rng = np.random.default_rng(1000 * ni + 10 * nb + G)
+    q = np.array(ctx.primes[:limbs], dtype=np.uint64).reshape(1, limbs, 1)
+    pts = _residues(rng, (G * nb, limbs, ctx.N), q)
+    babies = _residues(rng, (nb, 2, ni, limbs, ctx.N), q.reshape(1, 1, 1, limbs, 1))
+    # every product at its largest, and zeros
+    pts[:, :, :3] = np.array([p - 1 for p in ctx.primes[:limbs]], dtype=np.uint64).reshape(1, limbs, 1)
+    babies[..., :2] = np.array([p - 1 for p in ctx.primes[:limbs]], dtype=np.uint64).reshape(1, 1, 1, limbs, 1)
+    babies[..., 2] = 0
+    buf = torch.zeros(pts.size + 2, dtype=torch.uint64, device="cuda")
+    buf.view(torch.int64)[offset:offset + pts.size].copy_(torch.from_numpy(pts.view(np.int64)).reshape(-1))
+    tp = buf[offset:offset + pts.size].view(pts.shape)
+    bt = torch.from_numpy(babies).cuda()
+    res = ctx.bsgs_mac([bt[b, 0] for b in range(nb)], [bt[b, 1] for b in range(nb)], tp, limbs, G).cpu().numpy()
+    for i in range(ni):
+        want = orc.bsgs_mac(limbs, nb, G, pts, np.ascontiguousarray(babies[:, :, i]))
+        assert np.array_equal(res[:, :, i], want), f"input {i}"
+
+
+@pytest.mark.parametrize("ni,nb,G,limbs", [(8, 16, 16, 2), (7, 15, 15, 1), (5, 16, 32, 1), (15, 31, 30, 1),
+                                           (9, 48, 17, 1), (16, 64, 16, 1), (13, 33, 27, 1)])
+def test_matrix_core_tiles(env, ni, nb, G, limbs):
+    _check(env, ni, nb, G, limbs)
+
+
+@pytest.mark.parametrize("ni,nb,G,limbs", [(1, 9, 8, 2), (2, 3, 9, 1), (3, 8, 7, 1), (4, 2, 16, 1), (5, 8, 8, 1),
+                                           (10, 7, 1, 1)])
+def test_vector_tiles(env, ni, nb, G, limbs):
+    _check(env, ni, nb, G, limbs)
+
+
+def test_rows_that_are_not_16_byte_aligned(env):
+    """A shape of the matrix-core kernel whose plaintexts start at an odd word."""
+    _check(env, 8, 16, 16, 1, offset=1)
