@@ -6,7 +6,8 @@
 // method that the giant steps then rotate and add (exact-residue semantics of
 // bench/cmp/kernels/holmes_mac.cu:8-12, multi-input tiling of holmes_mac.cu:108-190).
 //
-// A thread owns one coefficient of one limb and
+// Two kernels: with enough inputs, giants and babies to fill its 16 x 16 x 16 tiles the matrix-core MAC
+// of mac_mx.hpp, else k_bsgs_mac on the VALU.  In the latter a thread owns one coefficient of one limb and
 // a TI x 8 tile of (input, giant) accumulators for both components: per baby step it reads 8 plaintext
 // words and 2 TI baby words for 16 TI products (the next step's words are loaded while the current step
 // computes), so plaintexts stream once per input tile and babies once per giant tile.  Up to 3 inputs HBM
@@ -19,6 +20,7 @@
 
 #include "../../include/holmes_ckks.h"
 #include "internal.hpp"
+#include "mac_mx.hpp"
 #include "wide.hpp"
 #include "modarith64.hpp"
 
@@ -154,6 +156,42 @@ __global__ __launch_bounds__(kMacThreads) void k_bsgs_mac(uint64_t* __restrict__
   }
 }
 
+// The matrix-core MAC's arithmetic for primes below 2^50 (mac_mx.hpp): canonical words below 2^50 have
+// seven balanced digits (the top one at most 4).  The byte-pair sums a_k (|a_k| < 2^29, a_6 the top
+// digit's own sum, below 2^9) give d0 + 2^32 d1 + 2^64 d2 with |d0|, |d1| < 2^46 and |d2| < 2^46:
+// 2^32 d1 is exact, its quotient rint(2^32 d1 / p) leaves an exact remainder within 0.51 p, and
+// d2 * (2^64 mod p) is one lazy product within 0.51 p.  Four steps of 16 babies stay below
+// 4 (2^46 + 1.1 p) < 2^53, so the running sum is reduced once, in finish().
+struct MxFp {
+  static constexpr int ND = 7;
+  typedef DevTables Tables;
+  typedef double Acc;
+  struct Consts {
+    double p, pinv, k32;
+    __device__ __forceinline__ void load(const DevTables& T, int pi) {
+      p = T.p[pi];
+      pinv = T.pinv[pi];
+      k32 = 4294967296.0 * pinv;
+    }
+  };
+  static __device__ __forceinline__ uint64_t digits(uint64_t x) {
+    constexpr uint64_t M = 0x0080808080808080ULL;
+    return (x + M) ^ M;
+  }
+  static __device__ __forceinline__ Acc zero() { return 0.0; }
+  static __device__ __forceinline__ void add(Acc& x, const int (&a)[ND], const Consts& C) {
+    const double d0 = __builtin_fma(65536.0, (double)a[1], (double)a[0]);
+    const double d1 = __builtin_fma(65536.0, (double)a[3], (double)a[2]);
+    const double d2 = __builtin_fma(4294967296.0, (double)a[6], __builtin_fma(65536.0, (double)a[5], (double)a[4]));
+    const double u = d1 + __builtin_fma(-__builtin_rint(d2 * C.k32), C.p, d2 * 4294967296.0);
+    x += d0 + __builtin_fma(-__builtin_rint(u * C.k32), C.p, u * 4294967296.0);
+  }
+  static __device__ __forceinline__ uint64_t finish(Acc x, const Consts& C) {
+    const double r = reduce(x, C.p, C.pinv);  // within p/2 + 2
+    return d2u(r < 0.0 ? r + C.p : r);
+  }
+};
+
 // ----------------------------------------------------------------- the sidecar-shaped MAC
 // holmes_mac_multi's layout (bench/cmp/kernels/holmes_mac.cu:359-402): one device pointer per input to
 // its baby basis [nb][>= limbs][N] (baby stride bstride words), plaintext rows [groups * nb][>= limbs][N]
@@ -273,6 +311,14 @@ extern "C" int hck_bsgs_mac(const hck_context* ctx, int limbs, const int* prime_
     if (!baby_c0[b] || !baby_c1[b]) return HCK_ERR_ARG;
     bp.c0[b] = baby_c0[b];
     bp.c1[b] = baby_c1[b];
+  }
+  if (hck::mx_pays(inputs, babies, giants)) {
+    hck::MxArgs A = hck::mx_args(limbs, mp.prime, inputs, babies, giants, baby_c0, baby_c1, baby_stride, pts, pt_stride, res);
+    if (hck::mx_aligned(A)) {
+      hck::mx_launch<hck::MxFp>(A, ctx->dev, (hipStream_t)stream);
+      HCK_CHECK_LAUNCH();
+      return HCK_OK;
+    }
   }
   const int units_per_limb = hck::kN / hck::kMacThreads;
   const int total_units = limbs * units_per_limb;

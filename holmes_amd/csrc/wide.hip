@@ -19,6 +19,7 @@
 
 #include "../../include/holmes_ckks.h"
 #include "internal.hpp"
+#include "mac_mx.hpp"
 #include "modarith64.hpp"
 #include "wide.hpp"
 #include "wide_dev.hpp"
@@ -941,6 +942,34 @@ __global__ __launch_bounds__(kWMacThreads) void wk_bsgs_mac30(const WMac P, long
   }
 }
 
+// The matrix-core MAC's arithmetic for primes below 2^60 (mac_mx.hpp): canonical words have eight balanced
+// digits.  The byte-pair sums a_k (|a_k| < 2^30) add up to V = sum_k 2^(16 k) a_k = sum_b x_b w_b, which
+// is not negative and below 16 p^2: with a residue added it stays below p 2^64 (16 p + 1 < 2^64), so one
+// Montgomery fold per 16 babies gives the canonical residue.
+struct MxWide {
+  static constexpr int ND = 8;
+  typedef WideTables Tables;
+  typedef u64 Acc;
+  struct Consts {
+    u64 p, mneg, r, rs;
+    __device__ __forceinline__ void load(const WideTables& T, int pi) {
+      p = T.p[pi];
+      mneg = T.mneg[pi];
+      r = T.r64[pi];
+      rs = T.r64_s[pi];
+    }
+  };
+  static __device__ __forceinline__ u64 digits(u64 x) { return (x + kDigitBias) ^ kDigitBias; }
+  static __device__ __forceinline__ Acc zero() { return 0; }
+  static __device__ __forceinline__ void add(Acc& x, const int (&a)[ND], const Consts& C) {
+    auto pair = [&](int k) { return (long long)a[k] + ((long long)a[k + 1] << 16); };  // |.| < 2^46.1
+    const long long s0 = pair(0), s1 = pair(2), s2 = pair(4), s3 = pair(6);
+    const u128 v = (u128)((__int128)s0 + ((__int128)s1 << 32) + ((__int128)(s2 + (s3 << 32)) << 64));
+    x = wfold128(v + x, C.p, C.mneg, C.r, C.rs);
+  }
+  static __device__ __forceinline__ u64 finish(Acc x, const Consts&) { return x; }
+};
+
 // ---------------------------------------------------------------------------------------- encode
 constexpr double kWideEncodeCap = 2305843009213693952.0;  // 2^61, as the FP64 path
 
@@ -1808,6 +1837,14 @@ int wide_bsgs_mac(const hck_context* c, int limbs, const int* prime_idx, int inp
   const long long units_padded = ((long long)total_units + kXcds - 1) / kXcds * kXcds;
   bool split = true;  // the split MAC needs every prime of the launch below 2^60
   for (int l = 0; l < limbs; ++l) split = split && c->primes[prime_idx[l]] < (1ULL << 60);
+  if (split && mx_pays(inputs, babies, giants)) {
+    MxArgs A = mx_args(limbs, pm.prime, inputs, babies, giants, baby_c0, baby_c1, baby_stride, pts, pt_stride, res);
+    if (mx_aligned(A)) {
+      mx_launch<MxWide>(A, c->wide->t, s);
+      HCK_CHECK_LAUNCH();
+      return HCK_OK;
+    }
+  }
   if (split) {
     const int tiles_i = (inputs + kSTI - 1) / kSTI, tiles_g = (giants + kSTG - 1) / kSTG;
     const long long blocks = units_padded * tiles_i * tiles_g;
