@@ -77,10 +77,24 @@ __host__ __device__ __forceinline__ uint64_t submod64(uint64_t a, uint64_t c, ui
 // Shoup's companion of a constant c < p: floor(c 2^64 / p).  Host only (one 128-bit division).
 inline uint64_t shoup_companion(uint64_t c, uint64_t p) { return (uint64_t)(((u128_t)c << 64) / p); }
 
-// a * c mod p in [0, 2p) with c's companion (Shoup): q = floor(a c' / 2^64), r = a c - q p.
+// add + (a * c mod p in [0, 2p)) with c's companion (Shoup): q = floor(a c' / 2^64), r = a c - q p, all
+// modulo 2^64.  Written in 32-bit words as a c + q (2^64 - p) + add: the two low products and the
+// addend share one chain of multiply-adds and the four cross products one sum, 15 instructions where
+// two 64-bit products, a subtraction and an addition take 19.
+__host__ __device__ __forceinline__ uint64_t mulshoup_add(uint64_t a, uint64_t c, uint64_t cs, uint64_t p,
+                                                          uint64_t add) {
+  const uint64_t q = (uint64_t)(((u128_t)a * cs) >> 64), np = 0 - p;
+  const uint32_t al = (uint32_t)a, ah = (uint32_t)(a >> 32), cl = (uint32_t)c, ch = (uint32_t)(c >> 32);
+  const uint32_t ql = (uint32_t)q, qh = (uint32_t)(q >> 32), nl = (uint32_t)np, nh = (uint32_t)(np >> 32);
+  uint64_t t = (uint64_t)al * cl + add;
+  t += (uint64_t)ql * nl;
+  const uint32_t h = (uint32_t)(t >> 32) + al * ch + ah * cl + ql * nh + qh * nl;
+  return ((uint64_t)h << 32) | (uint32_t)t;
+}
+
+// a * c mod p in [0, 2p) (Shoup).
 __host__ __device__ __forceinline__ uint64_t mulshoup_lazy(uint64_t a, uint64_t c, uint64_t cs, uint64_t p) {
-  const uint64_t q = (uint64_t)(((u128_t)a * cs) >> 64);
-  return a * c - q * p;
+  return mulshoup_add(a, c, cs, p, 0);
 }
 
 }  // namespace hck

@@ -9,6 +9,22 @@
 
 namespace hck {
 
+// The compiler must not see through the value (a constant kept in registers as it is).
+__device__ __forceinline__ uint64_t opaque(uint64_t v) {
+  asm("" : "+v"(v));
+  return v;
+}
+__device__ __forceinline__ uint64_t opaque_s(uint64_t v) {  // a value that is uniform over the wave
+  asm("" : "+s"(v));
+  return v;
+}
+// x - c where that is not negative, else x, for |x - c| < 2^63; nc = opaque(2^64 - c).  The sum with nc is
+// one instruction and the sign one comparison: four instructions, where comparing and subtracting takes
+// five and a carry.
+__device__ __forceinline__ uint64_t wsub_if(uint64_t x, uint64_t nc) {
+  const uint64_t d = x + nc;
+  return (long long)d < 0 ? x : d;
+}
 __device__ __forceinline__ uint64_t wadd(uint64_t a, uint64_t b, uint64_t p) {
   const uint64_t s = a + b;
   return s >= p ? s - p : s;

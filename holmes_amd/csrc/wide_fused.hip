@@ -60,21 +60,20 @@ __device__ __forceinline__ uint32_t gal_of(const WGalF& G, int b) { return G.per
 // 64-bit v), so each stage raises the bound by 2p.  A forward pass of four stages takes words below 8p
 // to words below 16p (<= 2^64 for p < 2^60: wide_fused_ok) and subtracts 8p once at its end
 // (w_fwd_end), so every forward pass's outputs, and the transform's, lie below 8p.
-// Gentleman-Sande (u, v) -> (u + v, (u - v) w), inputs and outputs below 2p.  p2 = 2p.
+// Gentleman-Sande (u, v) -> (u + v, (u - v) w), inputs and outputs below 2p.  p2 = 2p, n2 = -2p and
+// n8 = -8p are opaque.
 __device__ __forceinline__ void w_ct(u64& u, u64& v, u64 w, u64 ws, u64 p, u64 p2) {
   const u64 a = u;
-  const u64 y = mulshoup_lazy(v, w, ws, p);
-  u = a + y;
-  v = a - y + p2;
+  u = mulshoup_add(v, w, ws, p, a);
+  v = (a << 1) + p2 - u;
 }
-__device__ __forceinline__ void w_fwd_end(u64 (&x)[16], u64 p) {
-  const u64 p8 = 8 * p;
+__device__ __forceinline__ void w_fwd_end(u64 (&x)[16], u64 n8) {
 #pragma unroll
-  for (int k = 0; k < 16; ++k) x[k] = x[k] >= p8 ? x[k] - p8 : x[k];
+  for (int k = 0; k < 16; ++k) x[k] = wsub_if(x[k], n8);
 }
-__device__ __forceinline__ void w_gs(u64& u, u64& v, u64 w, u64 ws, u64 p, u64 p2) {
-  const u64 a = u, b = v, s = a + b;
-  u = s >= p2 ? s - p2 : s;
+__device__ __forceinline__ void w_gs(u64& u, u64& v, u64 w, u64 ws, u64 p, u64 p2, u64 n2) {
+  const u64 a = u, b = v;
+  u = wsub_if(a + b, n2);
   v = mulshoup_lazy(a - b + p2, w, ws, p);
 }
 
@@ -83,6 +82,7 @@ __device__ __forceinline__ void w_gs(u64& u, u64& v, u64 w, u64 ws, u64 p, u64 p
 // j + 16k (group k >> (4 - l)), layout B rows 16j + k (group (j << (l - 4)) + (k >> (8 - l))).
 __device__ __forceinline__ void wcol_fwd_lo(u64 (&x)[16], const u64* __restrict__ tw, const u64* __restrict__ tws,
                                             u64 p) {
+  const u64 p2 = opaque(2 * p);
 #pragma unroll
   for (int l = 0; l < 4; ++l) {
     const int h = 8 >> l;
@@ -90,14 +90,15 @@ __device__ __forceinline__ void wcol_fwd_lo(u64 (&x)[16], const u64* __restrict_
     for (int k = 0; k < 16; ++k) {
       if (k & h) continue;
       const int wi = (1 << l) + (k >> (4 - l));
-      w_ct(x[k], x[k + h], tw[wi], tws[wi], p, 2 * p);
+      w_ct(x[k], x[k + h], tw[wi], tws[wi], p, p2);
     }
   }
-  w_fwd_end(x, p);
+  w_fwd_end(x, opaque(0 - 8 * p));
 }
 
 __device__ __forceinline__ void wcol_fwd_hi(u64 (&x)[16], int j, const u64* __restrict__ tw,
                                             const u64* __restrict__ tws, u64 p) {
+  const u64 p2 = opaque(2 * p);
 #pragma unroll
   for (int l = 4; l < 8; ++l) {
     const int h = 128 >> l;
@@ -105,14 +106,15 @@ __device__ __forceinline__ void wcol_fwd_hi(u64 (&x)[16], int j, const u64* __re
     for (int k = 0; k < 16; ++k) {
       if (k & h) continue;
       const int wi = (1 << l) + (j << (l - 4)) + (k >> (8 - l));
-      w_ct(x[k], x[k + h], tw[wi], tws[wi], p, 2 * p);
+      w_ct(x[k], x[k + h], tw[wi], tws[wi], p, p2);
     }
   }
-  w_fwd_end(x, p);
+  w_fwd_end(x, opaque(0 - 8 * p));
 }
 
 __device__ __forceinline__ void wcol_inv_hi(u64 (&x)[16], int j, const u64* __restrict__ tw,
                                             const u64* __restrict__ tws, u64 p) {
+  const u64 p2 = opaque(2 * p), n2 = opaque(0 - 2 * p);
 #pragma unroll
   for (int l = 7; l >= 4; --l) {
     const int h = 128 >> l;
@@ -120,7 +122,7 @@ __device__ __forceinline__ void wcol_inv_hi(u64 (&x)[16], int j, const u64* __re
     for (int k = 0; k < 16; ++k) {
       if (k & h) continue;
       const int wi = (1 << l) + (j << (l - 4)) + (k >> (8 - l));
-      w_gs(x[k], x[k + h], tw[wi], tws[wi], p, 2 * p);
+      w_gs(x[k], x[k + h], tw[wi], tws[wi], p, p2, n2);
     }
   }
 }
@@ -129,6 +131,7 @@ __device__ __forceinline__ void wcol_inv_hi(u64 (&x)[16], int j, const u64* __re
 // n0 = N^-1 hinv, n1 = N^-1 psi_rev_inv[1] hinv (WideConv::inv_n0 / inv_n1); inputs below 2p
 __device__ __forceinline__ void wcol_inv_lo(u64 (&x)[16], const u64* __restrict__ tw, const u64* __restrict__ tws,
                                             u64 n0, u64 n0s, u64 n1, u64 n1s, u64 p) {
+  const u64 p2 = opaque(2 * p), n2 = opaque(0 - 2 * p);
 #pragma unroll
   for (int l = 3; l >= 1; --l) {
     const int h = 8 >> l;
@@ -136,7 +139,7 @@ __device__ __forceinline__ void wcol_inv_lo(u64 (&x)[16], const u64* __restrict_
     for (int k = 0; k < 16; ++k) {
       if (k & h) continue;
       const int wi = (1 << l) + (k >> (4 - l));
-      w_gs(x[k], x[k + h], tw[wi], tws[wi], p, 2 * p);
+      w_gs(x[k], x[k + h], tw[wi], tws[wi], p, p2, n2);
     }
   }
 #pragma unroll
@@ -154,6 +157,7 @@ __device__ __forceinline__ void wcol_inv_lo(u64 (&x)[16], const u64* __restrict_
 // stages' root addresses cost a few registers when the compiler hoists them out of a digit loop.
 __device__ __forceinline__ void wrow_fwd_lo(u64 (&x)[16], int b, const u64* __restrict__ tw,
                                             const u64* __restrict__ tws, u64 p) {
+  const u64 p2 = opaque_s(2 * p);
 #pragma unroll
   for (int l = 8; l < 12; ++l) {
     const int h = 2048 >> l;
@@ -163,14 +167,15 @@ __device__ __forceinline__ void wrow_fwd_lo(u64 (&x)[16], int b, const u64* __re
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
       if (k & h) continue;
-      w_ct(x[k], x[k + h], t[k >> (12 - l)], ts[k >> (12 - l)], p, 2 * p);
+      w_ct(x[k], x[k + h], t[k >> (12 - l)], ts[k >> (12 - l)], p, p2);
     }
   }
-  w_fwd_end(x, p);
+  w_fwd_end(x, opaque_s(0 - 8 * p));
 }
 
 __device__ __forceinline__ void wrow_fwd_hi(u64 (&x)[16], int b, int j, const u64* __restrict__ tw,
                                             const u64* __restrict__ tws, u64 p) {
+  const u64 p2 = opaque_s(2 * p);
 #pragma unroll
   for (int l = 12; l < 16; ++l) {
     const int h = 32768 >> l;
@@ -180,14 +185,15 @@ __device__ __forceinline__ void wrow_fwd_hi(u64 (&x)[16], int b, int j, const u6
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
       if (k & h) continue;
-      w_ct(x[k], x[k + h], t[k >> (16 - l)], ts[k >> (16 - l)], p, 2 * p);
+      w_ct(x[k], x[k + h], t[k >> (16 - l)], ts[k >> (16 - l)], p, p2);
     }
   }
-  w_fwd_end(x, p);
+  w_fwd_end(x, opaque_s(0 - 8 * p));
 }
 
 __device__ __forceinline__ void wrow_inv_hi(u64 (&x)[16], int b, int j, const u64* __restrict__ tw,
                                             const u64* __restrict__ tws, u64 p) {
+  const u64 p2 = opaque_s(2 * p), n2 = opaque_s(0 - 2 * p);
 #pragma unroll
   for (int l = 15; l >= 12; --l) {
     const int h = 32768 >> l;
@@ -197,13 +203,14 @@ __device__ __forceinline__ void wrow_inv_hi(u64 (&x)[16], int b, int j, const u6
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
       if (k & h) continue;
-      w_gs(x[k], x[k + h], t[k >> (16 - l)], ts[k >> (16 - l)], p, 2 * p);
+      w_gs(x[k], x[k + h], t[k >> (16 - l)], ts[k >> (16 - l)], p, p2, n2);
     }
   }
 }
 
 __device__ __forceinline__ void wrow_inv_lo(u64 (&x)[16], int b, const u64* __restrict__ tw,
                                             const u64* __restrict__ tws, u64 p) {
+  const u64 p2 = opaque_s(2 * p), n2 = opaque_s(0 - 2 * p);
 #pragma unroll
   for (int l = 11; l >= 8; --l) {
     const int h = 2048 >> l;
@@ -213,7 +220,7 @@ __device__ __forceinline__ void wrow_inv_lo(u64 (&x)[16], int b, const u64* __re
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
       if (k & h) continue;
-      w_gs(x[k], x[k + h], t[k >> (12 - l)], ts[k >> (12 - l)], p, 2 * p);
+      w_gs(x[k], x[k + h], t[k >> (12 - l)], ts[k >> (12 - l)], p, p2, n2);
     }
   }
 }
