@@ -51,6 +51,15 @@ __device__ __forceinline__ uint64_t wmont(uint64_t x, uint64_t k, uint64_t p, ui
   return th + (uint64_t)(((u128_t)m * p) >> 64) + (tl != 0 ? 1 : 0);
 }
 
+// x k 2^-64 mod p as a signed word in (-p, x k / 2^64): t - m p is a multiple of 2^64 for m = t p^-1 (pi64 =
+// p^-1 mod 2^64), its high word the difference of the high words.  No carry to form and nothing to
+// reduce per product: sums of a few are brought back together.
+__device__ __forceinline__ long long wmont_s(uint64_t x, uint64_t k, uint64_t p, uint64_t pi64) {
+  const u128_t t = (u128_t)x * k;
+  const uint64_t m = (uint64_t)t * pi64;
+  return (long long)((uint64_t)(t >> 64) - (uint64_t)(((u128_t)m * p) >> 64));
+}
+
 // t mod p for t < p 2^64: Montgomery's reduction (t 2^-64, below 2p), then the product with 2^64 mod p
 // (r = 2^64 mod p, rs its Shoup companion); canonical result.
 __device__ __forceinline__ uint64_t wfold128(u128_t t, uint64_t p, uint64_t mneg, uint64_t r, uint64_t rs) {

@@ -438,8 +438,12 @@ __global__ __launch_bounds__(kT, 2) void wf_cols_mconv(const WConvArgs A, WideTa
 // ----------------------------------------------------------------- inner product of one tile
 // sb / sa = sum_j x_j key_j[comp] mod p over the digits j of item b, extended limb e (prime pi), row
 // group rg: x_j the NTT rows pass of T2 digit j (below 8p), or, for the digit that holds limb e, d
-// itself read through sigma_g.  Montgomery products summed below 2p, then one product by 2^64 mod p:
-// canonical results.
+// itself read through sigma_g (taken first).  Signed Montgomery products (wmont_s) summed without a
+// reduction, then one product by 2^64 mod p: canonical results.  A term lies in (-p, p / 2) (x < 8p, k < p
+// < 2^60): after four of them on sums in [0, 4p) the sums lie in (-4p, 6p), where wsum_back() brings
+// them back (6p < 2^63).
+// A transform leaves its result in S, so that both key components and the next digit's tile are in
+// flight while the products are formed.
 struct WIp {
   const u64* d;
   long long d_stride;
@@ -448,51 +452,117 @@ struct WIp {
   int ell, beta, L, K, alpha, beta_max;
 };
 
-// FINISH = false leaves the sums in the Montgomery domain (x k 2^-64, below 2p) and INIT = false adds to
-// them: the grouped kernel runs several items' inner products into one pair of sums.
-template <bool INIT = true, bool FINISH = true>
-__device__ __forceinline__ void wtile_ip(u64 (&sb)[16], u64 (&sa)[16], u64 (&x)[16], const WIp& I, int b, int e,
-                                         int pi, int rg, uint32_t g, u64* S, const u64* __restrict__ tw,
+// sums in (-4p, 6p) -> [0, 4p)
+__device__ __forceinline__ void wsum_back(u64 (&s)[16], u64 p) {
+  const u64 p4 = opaque_s(4 * p), n4 = opaque_s(0 - 4 * p);
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+    const u64 lo = s[k] + p4, hi = s[k] + n4;
+    s[k] = (long long)s[k] < 0 ? lo : (long long)hi < 0 ? s[k] : hi;
+  }
+}
+// sums in (-4p, 6p), scaled by 2^64 mod p: canonical
+__device__ __forceinline__ void wsum_finish(u64 (&s)[16], u64 p, u64 r, u64 rs) {
+  const u64 p4 = opaque_s(4 * p);
+#pragma unroll
+  for (int k = 0; k < 16; ++k) s[k] = wmulc(s[k] + p4, r, rs, p);
+}
+constexpr int kSumTerms = 4;  // terms between two wsum_back
+
+__device__ __forceinline__ void wkeys(u64 (&kb)[16], u64 (&ka)[16], const u64* __restrict__ kp, long long comp) {
+#pragma unroll
+  for (int k = 0; k < 16; ++k) kb[k] = kp[16 * k];
+#pragma unroll
+  for (int k = 0; k < 16; ++k) ka[k] = kp[comp + 16 * k];
+}
+
+// cnt: the terms on sb since the last wsum_back (uniform).  FINISH = false leaves the sums in the
+// Montgomery domain and INIT = false adds to them: the grouped kernel runs several items' inner
+// products into one pair of sums.
+template <bool INIT = true, bool FINISH = true, bool PIPE = true>
+__device__ __forceinline__ void wtile_ip(u64 (&sb)[16], u64 (&sa)[16], u64 (&x)[16], int& cnt, const WIp& I, int b,
+                                         int e, int pi, int rg, uint32_t g, u64* S, const u64* __restrict__ tw,
                                          const u64* __restrict__ tws, const WideTables& T) {
-  const u64 p = T.p[pi], p2 = 2 * p, mneg = T.mneg[pi];
+  const u64 p = T.p[pi], pi64 = opaque_s(0 - T.mneg[pi]);
+  const RowMap mt = map_t(), mn = map_n();
   const int ext_l = I.ell + I.K;
   const long long comp = (long long)I.beta_max * (I.L + I.K) * kN;
-  const int own = e < I.ell ? e / I.alpha : -1;
+  const int own = e < I.ell ? e / I.alpha : -1, n2 = I.beta - (own >= 0 ? 1 : 0);
   const long long na = nat_a(rg);
   const u64* t2b = I.t2 + ((long long)b * I.beta * ext_l + e) * kN;
-  // one key component at a time: the 16 words of the other are not live across the products
-  auto mac = [&](u64 (&acc)[16], const u64* __restrict__ kp) {
-    u64 kw[16];
-#pragma unroll
-    for (int k = 0; k < 16; ++k) kw[k] = kp[16 * k];
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const u64 v = acc[k] + wmont(x[k], kw[k], p, mneg);  // below 3.5p
-      acc[k] = v >= p2 ? v - p2 : v;
+  const u64* kp = I.key + (long long)pi * kN + na;
+  const long long kstep = (long long)(I.L + I.K) * kN;
+  auto digit = [&](int n) { return own >= 0 && n >= own ? n + 1 : n; };
+  auto tick = [&]() {
+    if (cnt == kSumTerms) {
+      wsum_back(sb, p);
+      wsum_back(sa, p);
+      cnt = 0;
     }
+    ++cnt;
   };
+  u64 kb[16], ka[16];
   if constexpr (INIT) {
+    cnt = 0;
 #pragma unroll
     for (int k = 0; k < 16; ++k) sb[k] = sa[k] = 0;
   }
-  for (int jd = 0; jd < I.beta; ++jd) {
-    if (jd == own) {
-      load_gal_raw(x, I.d + (long long)b * I.d_stride + (long long)e * kN, na, g);
-    } else {
-      load_t(x, t2b + (long long)jd * ext_l * kN, rg);
-      wrows_fwd_t(x, rg, S, tw, tws, p);
-    }
-    const u64* kp = I.key + ((long long)jd * (I.L + I.K) + pi) * kN + na;
-    mac(sb, kp);
-    mac(sa, kp + comp);
-  }
-  if constexpr (!FINISH) return;
-  const u64 r = T.r64[pi], rs = T.r64_s[pi];
+  if constexpr (!PIPE) {
+    auto mac = [&](u64 (&acc)[16], const u64* __restrict__ kq) {
+      u64 kw[16];
 #pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    sb[k] = wmulc(sb[k], r, rs, p);
-    sa[k] = wmulc(sa[k], r, rs, p);
+      for (int k = 0; k < 16; ++k) kw[k] = kq[16 * k];
+#pragma unroll
+      for (int k = 0; k < 16; ++k) acc[k] += wmont_s(x[k], kw[k], p, pi64);
+    };
+    for (int jd = 0; jd < I.beta; ++jd) {
+      if (jd == own) {
+        load_gal_raw(x, I.d + (long long)b * I.d_stride + (long long)e * kN, na, g);
+      } else {
+        load_t(x, t2b + (long long)jd * ext_l * kN, rg);
+        wrows_fwd_t(x, rg, S, tw, tws, p);
+      }
+      tick();
+      mac(sb, kp + jd * kstep);
+      mac(sa, kp + jd * kstep + comp);
+    }
+    return;
   }
+  if (own >= 0) {
+    u64 xr[16];
+    load_gal_raw(xr, I.d + (long long)b * I.d_stride + (long long)e * kN, na, g);
+    wkeys(kb, ka, kp + own * kstep, comp);
+    if (n2 > 0) load_t(x, t2b + (long long)digit(0) * ext_l * kN, rg);
+    __builtin_amdgcn_sched_barrier(0);
+    tick();
+#pragma unroll
+    for (int k = 0; k < 16; ++k) sb[k] += wmont_s(xr[k], kb[k], p, pi64);
+#pragma unroll
+    for (int k = 0; k < 16; ++k) sa[k] += wmont_s(xr[k], ka[k], p, pi64);
+  } else if (n2 > 0) {
+    load_t(x, t2b + (long long)digit(0) * ext_l * kN, rg);
+  }
+  for (int n = 0; n < n2; ++n) {
+    wrow_fwd_lo(x, rg + 16 * mt.rb, tw, tws, p);
+    __syncthreads();  // the previous digit's reads of S are done
+    row_xchg<true, false>(x, S, mt, mn);
+    wrow_fwd_hi(x, rg + 16 * mn.rb, mn.j, tw, tws, p);
+#pragma unroll
+    for (int k = 0; k < 16; ++k) S[ridx(mn.rb, 16 * mn.j + k)] = x[k];
+    __syncthreads();
+    wkeys(kb, ka, kp + digit(n) * kstep, comp);
+    if (n + 1 < n2) load_t(x, t2b + (long long)digit(n + 1) * ext_l * kN, rg);
+    __builtin_amdgcn_sched_barrier(0);
+    tick();
+#pragma unroll
+    for (int k = 0; k < 16; ++k) sb[k] += wmont_s(S[ridx(mn.rb, mn.j + 16 * k)], kb[k], p, pi64);
+#pragma unroll
+    for (int k = 0; k < 16; ++k) sa[k] += wmont_s(S[ridx(mn.rb, mn.j + 16 * k)], ka[k], p, pi64);
+  }
+  __syncthreads();  // S is free for the caller
+  if constexpr (!FINISH) return;
+  wsum_finish(sb, p, T.r64[pi], T.r64_s[pi]);
+  wsum_finish(sa, p, T.r64[pi], T.r64_s[pi]);
 }
 
 // ----------------------------------------------------------------- K3: inner product, P limbs / ext
@@ -515,7 +585,8 @@ __global__ __launch_bounds__(kT, 2) void wf_rows_ip(const WIp I, const WGalF G, 
   WIp Ib = I;
   Ib.key = keys.k[b];
   u64 sb[16], sa[16], x[16];
-  wtile_ip(sb, sa, x, Ib, b, e, pi, rg, g, S, T.fwd + (size_t)pi * kN, T.fwd_s + (size_t)pi * kN, T);
+  int cnt;
+  wtile_ip(sb, sa, x, cnt, Ib, b, e, pi, rg, g, S, T.fwd + (size_t)pi * kN, T.fwd_s + (size_t)pi * kN, T);
   const long long na = nat_a(rg);
   if (ext_b) {
     if (e < I.ell && add) {
@@ -573,7 +644,7 @@ __global__ __launch_bounds__(kT, 2) void wf_rows_ip(const WIp I, const WGalF G, 
 // Output o (one tile of it per workgroup) is
 //   acc[o] + sum_m (P sigma_m(add[b]) + IP_b(sigma_m(d[b])), IP_a(sigma_m(d[b])))   over b = m * outputs + o,
 // each member with its own Galois element and key: the members' products and P sigma(add) (as the
-// Montgomery product by P mod p) run into one pair of lazy sums, scaled by 2^64 mod p once, so the
+// Montgomery product by P mod p) run into one pair of signed sums, scaled by 2^64 mod p once, so the
 // extended accumulator is read and written once per output.  Natural layout; ext may alias acc.
 __global__ __launch_bounds__(kT, 2) void wf_rows_ip_sum(const WIp I, const WGalF G, WKeysF keys, int outputs, int group,
                                                         int tiles, const u64* __restrict__ add, long long add_stride,
@@ -584,11 +655,12 @@ __global__ __launch_bounds__(kT, 2) void wf_rows_ip_sum(const WIp I, const WGalF
   if (id.tile >= tiles) return;
   const int o = id.b, e = id.tile >> 4, rg = id.tile & 15;
   const int pi = e < I.ell ? e : I.L + (e - I.ell);
-  const u64 p = T.p[pi], p2 = 2 * p, mneg = T.mneg[pi];
+  const u64 p = T.p[pi], pi64 = opaque_s(0 - T.mneg[pi]);
   const u64* tw = T.fwd + (size_t)pi * kN;
   const u64* tws = T.fwd_s + (size_t)pi * kN;
   const long long na = nat_a(rg);
   u64 sb[16], sa[16], x[16];
+  int cnt = 0;
 #pragma unroll
   for (int k = 0; k < 16; ++k) sb[k] = sa[k] = 0;
   for (int m = 0; m < group; ++m) {
@@ -596,23 +668,22 @@ __global__ __launch_bounds__(kT, 2) void wf_rows_ip_sum(const WIp I, const WGalF
     const uint32_t g = gal_of(G, b);
     WIp Ib = I;
     Ib.key = keys.k[b];
-    wtile_ip<false, false>(sb, sa, x, Ib, b, e, pi, rg, g, S, tw, tws, T);
+    wtile_ip<false, false, false>(sb, sa, x, cnt, Ib, b, e, pi, rg, g, S, tw, tws, T);
     if (e < I.ell && add) {
       load_gal_raw(x, add + (long long)b * add_stride + (long long)e * kN, na, g);
       const u64 pm = T.pmod[pi];
-#pragma unroll
-      for (int k = 0; k < 16; ++k) {
-        const u64 v = sb[k] + wmont(x[k], pm, p, mneg);  // below 3.5p
-        sb[k] = v >= p2 ? v - p2 : v;
+      if (cnt == kSumTerms) {
+        wsum_back(sb, p);
+        wsum_back(sa, p);
+        cnt = 0;
       }
+      ++cnt;
+#pragma unroll
+      for (int k = 0; k < 16; ++k) sb[k] += wmont_s(x[k], pm, p, pi64);
     }
   }
-  const u64 r = T.r64[pi], rs = T.r64_s[pi];
-#pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    sb[k] = wmulc(sb[k], r, rs, p);
-    sa[k] = wmulc(sa[k], r, rs, p);
-  }
+  wsum_finish(sb, p, T.r64[pi], T.r64_s[pi]);
+  wsum_finish(sa, p, T.r64[pi], T.r64_s[pi]);
   if (acc_b) {
     // read before the store below by the same thread: ext may alias acc
     const u64* ab = acc_b + (long long)o * acc_stride + (long long)e * kN + na;
@@ -654,7 +725,8 @@ __global__ __launch_bounds__(kT, 2) void wf_rows_ipq(const WIp I, const WGalF G,
   WIp Ib = I;
   Ib.key = keys.k[b];
   u64 sb[16], sa[16], x[16];
-  wtile_ip(sb, sa, x, Ib, b, i, i, rg, g, S, tw, tws, T);
+  int cnt;
+  wtile_ip(sb, sa, x, cnt, Ib, b, i, i, rg, g, S, tw, tws, T);
   const long long na = nat_a(rg);
   const u64 pv = T.pinv[i], pvs = T.pinv_s[i];
   auto finish = [&](u64 (&s)[16], int comp, const u64* addend, const u64* ac, u64* out) {
@@ -718,7 +790,8 @@ __global__ __launch_bounds__(kT, 2) void wf_rows_ipq_rs(const WIp I, const WGalF
   WIp Ib = I;
   Ib.key = keys.k[b];
   u64 sb[16], sa[16], x[16];
-  wtile_ip(sb, sa, x, Ib, b, i, i, rg, g, S, tw, tws, T);
+  int cnt;
+  wtile_ip(sb, sa, x, cnt, Ib, b, i, i, rg, g, S, tw, tws, T);
   const long long na = nat_a(rg);
   const u64 pv = T.pinv[i], pvs = T.pinv_s[i], ql = post.ql[i], qls = post.ql_s[i];
   const u64 r64 = T.r64[i], r64s = T.r64_s[i];
@@ -893,8 +966,7 @@ __global__ __launch_bounds__(kT) void wf_hoist_store(const u64* __restrict__ t2,
 }
 
 // Item b rotates input (src0 + b) % inputs by its Galois element: the inner product reads every digit
-// through sigma_g (ModUp commutes with sigma_g), with no row transform.  Montgomery products summed
-// below 2p, then one product by 2^64 mod p: canonical.
+// through sigma_g (ModUp commutes with sigma_g), with no row transform.  The sums as in wtile_ip.
 struct WHoist {
   const u64* digits;
   int inputs, src0;
@@ -902,34 +974,28 @@ struct WHoist {
 __device__ __forceinline__ void wtile_ip_h(u64 (&sb)[16], u64 (&sa)[16], u64 (&x)[16], const WHoist& H,
                                            const u64* __restrict__ key, int beta, int ell, int L, int K, int beta_max,
                                            int b, int e, int pi, int rg, uint32_t g, const WideTables& T) {
-  const u64 p = T.p[pi], p2 = 2 * p, mneg = T.mneg[pi];
+  const u64 p = T.p[pi], pi64 = opaque_s(0 - T.mneg[pi]);
   const int ext_l = ell + K, src = (H.src0 + b) % H.inputs;
   const long long comp = (long long)beta_max * (L + K) * kN;
   const long long na = nat_a(rg);
-  auto mac = [&](u64 (&acc)[16], const u64* __restrict__ kp) {
-    u64 kw[16];
-#pragma unroll
-    for (int k = 0; k < 16; ++k) kw[k] = kp[16 * k];
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const u64 v = acc[k] + wmont(x[k], kw[k], p, mneg);
-      acc[k] = v >= p2 ? v - p2 : v;
-    }
-  };
+  u64 kb[16], ka[16];
 #pragma unroll
   for (int k = 0; k < 16; ++k) sb[k] = sa[k] = 0;
   for (int jd = 0; jd < beta; ++jd) {
     load_gal_raw(x, H.digits + ((long long)(src * beta + jd) * ext_l + e) * kN, na, g);
-    const u64* kp = key + ((long long)jd * (L + K) + pi) * kN + na;
-    mac(sb, kp);
-    mac(sa, kp + comp);
-  }
-  const u64 r = T.r64[pi], rs = T.r64_s[pi];
+    wkeys(kb, ka, key + ((long long)jd * (L + K) + pi) * kN + na, comp);
+    __builtin_amdgcn_sched_barrier(0);
+    if (jd && jd % kSumTerms == 0) {
+      wsum_back(sb, p);
+      wsum_back(sa, p);
+    }
 #pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    sb[k] = wmulc(sb[k], r, rs, p);
-    sa[k] = wmulc(sa[k], r, rs, p);
+    for (int k = 0; k < 16; ++k) sb[k] += wmont_s(x[k], kb[k], p, pi64);
+#pragma unroll
+    for (int k = 0; k < 16; ++k) sa[k] += wmont_s(x[k], ka[k], p, pi64);
   }
+  wsum_finish(sb, p, T.r64[pi], T.r64_s[pi]);
+  wsum_finish(sa, p, T.r64[pi], T.r64_s[pi]);
 }
 
 // P limbs of hoisted rotations: the inner product's INTT rows pass into ACCP ([item][2][K]).
