@@ -73,9 +73,7 @@ __device__ __forceinline__ void gs_bf(double& u, double& v, const double w, doub
 }
 
 // ----------------------------------------------------------------- column transforms (16 threads)
-// forward stages 0..3 on layout A.  Inputs already within p/2 + 1 (REDUCED) skip the reduction
-// of stage 0; the bounds after stage 1 are then those of the reducing schedule (<= 2.15 p).
-template <bool REDUCED = false>
+// forward stages 0..3 on layout A (inputs within p/2 + 1)
 __device__ __forceinline__ void col_fwd_lo(double (&x)[16], const double* __restrict__ tw, double p, double pinv) {
 #pragma unroll
   for (int l = 0; l < 4; ++l) {
@@ -84,8 +82,8 @@ __device__ __forceinline__ void col_fwd_lo(double (&x)[16], const double* __rest
     for (int k = 0; k < 16; ++k) {
       if (k & h) continue;
       const double w = tw[(1 << l) + (k >> (4 - l))];
-      if ((l & 1) || (REDUCED && l == 0)) ct_bf<false>(x[k], x[k + h], w, p, pinv);
-      else ct_bf<true>(x[k], x[k + h], w, p, pinv);
+      if (fwd_reduces(l)) ct_bf<true>(x[k], x[k + h], w, p, pinv);
+      else ct_bf<false>(x[k], x[k + h], w, p, pinv);
     }
   }
 }
@@ -100,8 +98,8 @@ __device__ __forceinline__ void col_fwd_hi(double (&x)[16], int j, const double*
     for (int k = 0; k < 16; ++k) {
       if (k & h) continue;
       const double w = tw[(1 << l) + (j << (l - 4)) + (k >> (8 - l))];
-      if (l & 1) ct_bf<false>(x[k], x[k + h], w, p, pinv);
-      else ct_bf<true>(x[k], x[k + h], w, p, pinv);
+      if (fwd_reduces(l)) ct_bf<true>(x[k], x[k + h], w, p, pinv);
+      else ct_bf<false>(x[k], x[k + h], w, p, pinv);
     }
   }
 }
@@ -151,8 +149,8 @@ __device__ __forceinline__ void row_fwd_lo(double (&x)[16], int b, const double*
     for (int k = 0; k < 16; ++k) {
       if (k & h) continue;
       const double w = tw[(1 << l) + (b << (l - 8)) + (k >> (12 - l))];
-      if (l & 1) ct_bf<false>(x[k], x[k + h], w, p, pinv);
-      else ct_bf<true>(x[k], x[k + h], w, p, pinv);
+      if (fwd_reduces(l)) ct_bf<true>(x[k], x[k + h], w, p, pinv);
+      else ct_bf<false>(x[k], x[k + h], w, p, pinv);
     }
   }
 }
@@ -167,8 +165,8 @@ __device__ __forceinline__ void row_fwd_hi(double (&x)[16], int b, int j, const 
     for (int k = 0; k < 16; ++k) {
       if (k & h) continue;
       const double w = tw[(1 << l) + (b << (l - 8)) + (j << (l - 12)) + (k >> (16 - l))];
-      if (l & 1) ct_bf<false>(x[k], x[k + h], w, p, pinv);
-      else ct_bf<true>(x[k], x[k + h], w, p, pinv);
+      if (fwd_reduces(l)) ct_bf<true>(x[k], x[k + h], w, p, pinv);
+      else ct_bf<false>(x[k], x[k + h], w, p, pinv);
     }
   }
 }
@@ -375,7 +373,7 @@ __device__ __forceinline__ void cols_conv_body(const ConvArgs& A, int bx, int y,
         if (act) {
 #pragma unroll
           for (int k = 0; k < 16; ++k) x[u][k] = reduce(x[u][k], p[u], pinv[u]);
-          col_fwd_lo<true>(x[u], tw, p[u], pinv[u]);
+          col_fwd_lo(x[u], tw, p[u], pinv[u]);
         }
         col_a_to_b(x[u], RX, j);
         if (act) {
@@ -425,27 +423,23 @@ __device__ __forceinline__ uint64_t digit_word(double y) {
   return ((uint64_t)__double_as_longlong(t) + (M - 0x4338000000000000ULL)) ^ M;
 }
 
-// sum_c C_c 256^c mod p into [-p/2 - 1, p/2 + 1] (|C_c| < 2^20): lo = C_0..C_3 part (|lo| < 2^45),
-// hi = C_4..C_6 part (|hi| < 2^37), value lo + 2^32 hi.  hi 2^32 is exact; q = rint(hi 2^32 / p)
-// leaves |hi 2^32 - q p| <= 1.5 p (exact FMA), the sum with lo stays below 2^52, and reduce()
-// centers it.
+// sum_c C_c 256^c (+ r) mod p into [-p/2 - 1, p/2 + 1] (|C_c| < 2^20, |r| < 2^49): lo = C_0..C_3 part
+// (|lo| < 2^45) + r, hi = C_4..C_6 part (|hi| < 2^37), value lo + 2^32 hi.  The value is below 2^13 p
+// (56 digits times centered constants), so rint of its estimated quotient leaves it within p/2 + 1;
+// hi 2^32 - q p is then an integer below 2^51 and the FMA exact.  k32 = 2^32 / p.
 // The pairs a = C_0 + 256 C_1, b = C_2 + 256 C_3, d = C_4 + 256 C_5 and C_6 (each |.| < 2^29).
-__device__ __forceinline__ double mconv_fold(int a, int b, int d, int c6, double p, double pinv) {
-  const double lo = __builtin_fma(65536.0, (double)b, (double)a);
-  const double hi = __builtin_fma(65536.0, (double)c6, (double)d);
-  const double q = __builtin_rint(hi * (4294967296.0 * pinv));
-  const double r = __builtin_fma(-q, p, hi * 4294967296.0) + lo;
-  return reduce(r, p, pinv);
+__device__ __forceinline__ double mconv_fold_lohi(double lo, double hi, double p, double pinv, double k32) {
+  const double q = __builtin_rint(__builtin_fma(hi, k32, lo * pinv));
+  return __builtin_fma(-q, p, hi * 4294967296.0) + lo;
 }
-
-// mconv_fold with an integer addend r (|r| < 2^49) in the low part: |lo + r| < 2^50, and the
-// fold's final sum stays below 2^52.
-__device__ __forceinline__ double mconv_fold_add(int a, int b, int d, int c6, double r, double p, double pinv) {
-  const double lo = __builtin_fma(65536.0, (double)b, (double)a) + r;
-  const double hi = __builtin_fma(65536.0, (double)c6, (double)d);
-  const double q = __builtin_rint(hi * (4294967296.0 * pinv));
-  const double v = __builtin_fma(-q, p, hi * 4294967296.0) + lo;
-  return reduce(v, p, pinv);
+__device__ __forceinline__ double mconv_fold(int a, int b, int d, int c6, double p, double pinv, double k32) {
+  return mconv_fold_lohi(__builtin_fma(65536.0, (double)b, (double)a), __builtin_fma(65536.0, (double)c6, (double)d), p,
+                         pinv, k32);
+}
+__device__ __forceinline__ double mconv_fold_add(int a, int b, int d, int c6, double r, double p, double pinv,
+                                                 double k32) {
+  return mconv_fold_lohi(__builtin_fma(65536.0, (double)b, (double)a) + r,
+                         __builtin_fma(65536.0, (double)c6, (double)d), p, pinv, k32);
 }
 
 template <bool SEPX, int MI = kMItems>
@@ -529,7 +523,7 @@ __device__ __forceinline__ void cols_mconv_body(const ConvArgs& A, int bx, int y
       for (int r = 0; r < MI; ++r) {
         x[r][k] = r < mi ? mconv_fold(acc[0][r] + (int)((uint32_t)acc[1][r] << 8),
                                       acc[2][r] + (int)((uint32_t)acc[3][r] << 8),
-                                      acc[4][r] + (int)((uint32_t)acc[5][r] << 8), acc[6][r], p[r], pinv[r])
+                                      acc[4][r] + (int)((uint32_t)acc[5][r] << 8), acc[6][r], p[r], pinv[r], 4294967296.0 * pinv[r])
                          : 0.0;
         // the fold happens here, in its tile: sunk to its use in the transform, every tile's
         // accumulators would stay live at once
@@ -543,7 +537,7 @@ __device__ __forceinline__ void cols_mconv_body(const ConvArgs& A, int bx, int y
       if (r >= mi) break;  // uniform over the block
       const bool act = to[r] < nt;
       const double* __restrict__ tw = T.tw_fwd + (size_t)C.dst_prime[act ? to[r] : 0] * kN;
-      if (act) col_fwd_lo<true>(x[r], tw, p[r], pinv[r]);
+      if (act) col_fwd_lo(x[r], tw, p[r], pinv[r]);
       col_a_to_b(x[r], RX, j);
       if (act) {
         col_fwd_hi(x[r], j, tw, p[r], pinv[r]);
@@ -687,7 +681,8 @@ __device__ __forceinline__ void cols_mconv_rs_body(const ConvArgs& A, int bx, in
       for (int r = 0; r < MI; ++r) {
         x[r][k] = r < mi ? mconv_fold_add(acc[0][r] + (int)((uint32_t)acc[1][r] << 8),
                                           acc[2][r] + (int)((uint32_t)acc[3][r] << 8),
-                                          acc[4][r] + (int)((uint32_t)acc[5][r] << 8), acc[6][r], rz, p[r], pinv[r])
+                                          acc[4][r] + (int)((uint32_t)acc[5][r] << 8), acc[6][r], rz, p[r], pinv[r],
+                                          4294967296.0 * pinv[r])
                          : 0.0;
         asm volatile("" : "+v"(x[r][k]));
       }
@@ -699,7 +694,7 @@ __device__ __forceinline__ void cols_mconv_rs_body(const ConvArgs& A, int bx, in
       if (r >= mi) break;  // uniform over the block
       const bool act = to[r] < nt;
       const double* __restrict__ tw = T.tw_fwd + (size_t)C.dst_prime[act ? to[r] : 0] * kN;
-      if (act) col_fwd_lo<true>(x[r], tw, p[r], pinv[r]);
+      if (act) col_fwd_lo(x[r], tw, p[r], pinv[r]);
       col_a_to_b(x[r], RX, j);
       if (act) {
         col_fwd_hi(x[r], j, tw, p[r], pinv[r]);
@@ -783,8 +778,8 @@ __device__ __forceinline__ void row_fwd_lo_lds(double (&x)[16], const double* R,
     for (int k = 0; k < 16; ++k) {
       if (k & h) continue;
       const double w = R[(1 << (l - 8)) + (k >> (12 - l))];
-      if (l & 1) ct_bf<false>(x[k], x[k + h], w, p, pinv);
-      else ct_bf<true>(x[k], x[k + h], w, p, pinv);
+      if (fwd_reduces(l)) ct_bf<true>(x[k], x[k + h], w, p, pinv);
+      else ct_bf<false>(x[k], x[k + h], w, p, pinv);
     }
   }
 }
@@ -798,8 +793,8 @@ __device__ __forceinline__ void row_fwd_hi_lds(double (&x)[16], const double* R,
     for (int k = 0; k < 16; ++k) {
       if (k & h) continue;
       const double w = R[(1 << (l - 8)) + 16 * (k >> (16 - l)) + j];
-      if (l & 1) ct_bf<false>(x[k], x[k + h], w, p, pinv);
-      else ct_bf<true>(x[k], x[k + h], w, p, pinv);
+      if (fwd_reduces(l)) ct_bf<true>(x[k], x[k + h], w, p, pinv);
+      else ct_bf<false>(x[k], x[k + h], w, p, pinv);
     }
   }
 }
@@ -966,10 +961,10 @@ __device__ __forceinline__ void tile_ip_body(double (&sb)[16], double (&sa)[16],
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
       const double v = S[s_out(k)];
-      sb[k] += mulv(v, u2d(kb[k]), p, pinv);  // |v| <= 3.9p: |term| <= 2p
+      sb[k] += mulv(v, u2d(kb[k]), p, pinv);  // |v| <= 5.5p: |term| <= 2.6p
       sa[k] += mulv(v, u2d(ka[k]), p, pinv);
     }
-    if (n % 3 == 2) {  // <= p/2 + 1 + 3 * 2p (+ 0.9p for the own digit) < 8p <= 2^53 between reductions
+    if (n % 2 == 1 && n + 1 < I.nt2) {  // <= p/2 + 1 + 2 * 2.6p (+ 0.9p for the own digit) < 8p <= 2^53 between
 #pragma unroll
       for (int k = 0; k < 16; ++k) { sb[k] = reduce(sb[k], p, pinv); sa[k] = reduce(sa[k], p, pinv); }
     }
@@ -1114,7 +1109,7 @@ __device__ __forceinline__ void ipq_finish(double (&ip)[16], double (&x)[16], co
   double ad[16];
   if (add_limb) load_gal(ad, add_limb, na, g);
 #pragma unroll
-  for (int k = 0; k < 16; ++k) ip[k] = mulc(ip[k] - S[s_out(k)], pinv_P, p);  // |ip - v| <= 4.5 p: |r| <= 2.2 p
+  for (int k = 0; k < 16; ++k) ip[k] = mulc(ip[k] - S[s_out(k)], pinv_P, p);  // |ip - v| <= 6 p: |r| <= 2.8 p
   if (add_limb) {
 #pragma unroll
     for (int k = 0; k < 16; ++k) ip[k] += ad[k];
@@ -1122,7 +1117,7 @@ __device__ __forceinline__ void ipq_finish(double (&ip)[16], double (&x)[16], co
   if (acc_limb) {
     load_gal(ad, acc_limb, na, 1u);
 #pragma unroll
-    for (int k = 0; k < 16; ++k) ip[k] += ad[k];  // |r| <= 4.2 p
+    for (int k = 0; k < 16; ++k) ip[k] += ad[k];  // |r| <= 4.8 p
   }
 #pragma unroll
   for (int k = 0; k < 16; ++k) o[16 * k] = d2u(canon(ip[k], p, pinv));
@@ -1144,9 +1139,9 @@ __device__ __forceinline__ void ipq_finish_rs(double (&ip)[16], double (&x)[16],
   rows_fwd_lds(x, S, TW, p, pinv);
   if (next) load_t(x, next, rg);
 #pragma unroll
-  for (int k = 0; k < 16; ++k) ip[k] = mulc(ip[k], pinv_P, p) - S[s_out(k)];  // |.| <= p + 3.9 p
+  for (int k = 0; k < 16; ++k) ip[k] = mulc(ip[k], pinv_P, p) - S[s_out(k)];  // |.| <= 0.7 p + 5.5 p
   double ad[16];
-  if (px1) {  // the tensor term formed here: x1 y1 (+ x2 y2), each product within 0.875 p
+  if (px1) {  // the tensor term formed here: x1 y1 (+ x2 y2), each product within 0.875 p, the sum below 8 p
     double t[16];
     load_gal(ad, px1, na, 1u);
     load_gal(t, py1, na, 1u);
@@ -1167,7 +1162,7 @@ __device__ __forceinline__ void ipq_finish_rs(double (&ip)[16], double (&x)[16],
   if (acc_limb) {
     load_gal(ad, acc_limb, na, 1u);
 #pragma unroll
-    for (int k = 0; k < 16; ++k) ip[k] += ad[k];  // |.| <= 6.9 p
+    for (int k = 0; k < 16; ++k) ip[k] += ad[k];  // |.| <= 7.2 p with one of add and acc
   }
   if (!sub_limb && !twice && scalar == 0.0) {
 #pragma unroll
@@ -1175,7 +1170,7 @@ __device__ __forceinline__ void ipq_finish_rs(double (&ip)[16], double (&x)[16],
     return;
   }
 #pragma unroll
-  for (int k = 0; k < 16; ++k) {  // |r| <= 1.5 p: |2 r - sub + scalar| <= 5 p
+  for (int k = 0; k < 16; ++k) {  // |r| <= 2.5 p: |2 r - sub + scalar| <= 7 p
     const double r = mulc(ip[k], ql_inv, p);
     ip[k] = (twice ? 2.0 * r : r) + scalar;
   }
@@ -1410,7 +1405,7 @@ __global__ __launch_bounds__(kT) void k_ks_rows_finish(const double* __restrict_
   const TwPair pi_ = inv[i];
   uint64_t* o = out + (long long)pl * out_pstride + (long long)i * kN + na;
 #pragma unroll
-  for (int k = 0; k < 16; ++k) o[16 * k] = d2u(canon(mulc(a[k] - x[k], pi_, p), p, pinv));  // |a - x| <= 4.9 p
+  for (int k = 0; k < 16; ++k) o[16 * k] = d2u(canon(mulc(a[k] - x[k], pi_, p), p, pinv));  // |a - x| <= 6.5 p
 }
 
 // ----------------------------------------------------------------- NTT rows + canonical store
@@ -1860,7 +1855,7 @@ __global__ __launch_bounds__(kT) void k_lc_finish(const LcRsArgs A, int terms, c
   const double ad = ((add_mask >> g) & 1ull) ? u2d(A.add[i]) : 0.0;
   uint64_t* o = A.out[g] + (long long)i * kN + na;
 #pragma unroll
-  for (int k = 0; k < 16; ++k) o[16 * k] = d2u(canon(mulc(a[k] - x[k], qi, p) + ad, p, pinv));  // |a - x| <= 4.9 p
+  for (int k = 0; k < 16; ++k) o[16 * k] = d2u(canon(mulc(a[k] - x[k], qi, p) + ad, p, pinv));  // |a - x| <= 6.5 p
 }
 
 size_t lincomb_rescale_bytes(const hck_context* c, int ell, int groups) {

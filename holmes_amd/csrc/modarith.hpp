@@ -57,20 +57,18 @@ __device__ __forceinline__ double reduce(double x, double p, double pinv) {
   return __builtin_fma(-q, p, x);
 }
 
-// x mod p into [0, p) for exact |x| <= 2^53.
+// x mod p into [0, p) for exact |x| <= 2^53, and for any integer |x| <= 2^61 that is a double: the
+// centered remainder (exact, one FMA) lies strictly between -p and p.
 __device__ __forceinline__ double canon(double x, double p, double pinv) {
-  const double q = __builtin_floor(x * pinv);
-  double r = __builtin_fma(-q, p, x);
-  r = r < 0.0 ? r + p : r;
-  r = r >= p ? r - p : r;
-  return r;
+  const double r = reduce(x, p, pinv);
+  return r < 0.0 ? r + p : r;
 }
 
 // a * b mod p for a residue b in [0, p) without a stored companion: the quotient is estimated
 // from the product itself, q = rint(fl(a * b) * pinv).  fl(fl(a b) pinv) is within three
 // roundings of X = a b / p, so |q - X| <= 0.5 + |X| 3 2^-53, and with |X| < |a| = A p,
 //   |r| <= (0.5 + 0.375 A) p   (p < 2^50),
-// the bound of mulc.  For |a| <= 2^52 (A <= 4): |h - q p| <= 2p + 2^49 < 2^53, so the FMA is
+// the bound of mulc.  For |a| < 2^53 (A < 8): |h - q p| <= 3.5 p + 2^49 < 2^53, so the FMA is
 // exact and r == a b (mod p).  Twiddle tables store only w (8 bytes), and the product doubles as
 // the quotient's input: 6 FP64 operations.
 __device__ __forceinline__ double mulv(double a, double b, double p, double pinv) {
@@ -79,6 +77,14 @@ __device__ __forceinline__ double mulv(double a, double b, double p, double pinv
   const double l = __builtin_fma(a, b, -h);
   return __builtin_fma(-q, p, h) + l;
 }
+
+// The forward transform's stages that reduce their sum operand (stage l of 0 .. 15).  With A the largest
+// |x| / p, a stage (u, v) -> (u + w v, u - w v) takes A to 0.5 + 1.375 A, or to 1 + 0.375 A when it
+// reduces u.  From canonical words (A = 1) the column stages end at
+// 1.88 3.08 4.73 [2.78] 4.32 6.44 [3.42] 5.20 and the row stages at
+// 7.65 [3.87] 5.82 [3.19] 4.88 7.21 [3.71] 5.60; from centered words (A = 0.5) at 4.73 and 5.47.  Every
+// value stays below 8 p <= 2^53, so all of them are exact.
+constexpr bool fwd_reduces(int l) { return l == 3 || l == 6 || l == 9 || l == 11 || l == 14; }
 
 // Round half away from zero (llround semantics), written out: the library round() of this
 // toolchain does not send negative ties away from zero.  trunc, one exact subtraction and two

@@ -15,10 +15,8 @@
 // consecutive words.  Between the passes the limb is kept in HBM as signed-lazy doubles
 // (modarith.hpp), so only the final pass canonicalises.
 //
-// Lazy-reduction bounds (p < 2^50, mulv error model of modarith.hpp): forward stages reduce the
-// sum operand on even stages only; with B_e, B_o the bounds (in units of p) after even and odd
-// stages, B_e = 1 + 0.375 B_o and B_o = 0.5 + 1.375 B_e, so values stay below 2.45 p and 3.9 p
-// (< 2^52).  Inverse stages reduce every sum: values stay below 2 p.
+// Lazy-reduction bounds: modarith.hpp, fwd_reduces (forward).  Inverse stages reduce every sum: values
+// stay below 2 p.
 #include <hip/hip_runtime.h>
 
 #include "../../include/holmes_ckks.h"
@@ -87,8 +85,8 @@ __global__ __launch_bounds__(kThreads) void k_fwd_cols(const void* __restrict__ 
     for (int k = 0; k < 16; ++k) {
       if (k & h) continue;
       const double w = tw[(1 << l) + (k >> (4 - l))];
-      if (l & 1) ct<false>(x[k], x[k + h], w, p, pinv);
-      else ct<true>(x[k], x[k + h], w, p, pinv);
+      if (fwd_reduces(l)) ct<true>(x[k], x[k + h], w, p, pinv);
+      else ct<false>(x[k], x[k + h], w, p, pinv);
     }
   }
 #pragma unroll
@@ -104,8 +102,8 @@ __global__ __launch_bounds__(kThreads) void k_fwd_cols(const void* __restrict__ 
     for (int k = 0; k < 16; ++k) {
       if (k & h) continue;
       const double w = tw[(1 << l) + (j << (l - 4)) + (k >> (8 - l))];
-      if (l & 1) ct<false>(x[k], x[k + h], w, p, pinv);
-      else ct<true>(x[k], x[k + h], w, p, pinv);
+      if (fwd_reduces(l)) ct<true>(x[k], x[k + h], w, p, pinv);
+      else ct<false>(x[k], x[k + h], w, p, pinv);
     }
   }
 #pragma unroll
@@ -135,8 +133,8 @@ __global__ __launch_bounds__(kThreads) void k_fwd_rows(void* data, long long str
     for (int k = 0; k < 16; ++k) {
       if (k & h) continue;
       const double w = tw[(1 << l) + (b << (l - 8)) + (k >> (12 - l))];
-      if (l & 1) ct<false>(x[k], x[k + h], w, p, pinv);
-      else ct<true>(x[k], x[k + h], w, p, pinv);
+      if (fwd_reduces(l)) ct<true>(x[k], x[k + h], w, p, pinv);
+      else ct<false>(x[k], x[k + h], w, p, pinv);
     }
   }
 #pragma unroll
@@ -152,8 +150,8 @@ __global__ __launch_bounds__(kThreads) void k_fwd_rows(void* data, long long str
     for (int k = 0; k < 16; ++k) {
       if (k & h) continue;
       const double w = tw[(1 << l) + (b << (l - 8)) + (j << (l - 12)) + (k >> (16 - l))];
-      if (l & 1) ct<false>(x[k], x[k + h], w, p, pinv);
-      else ct<true>(x[k], x[k + h], w, p, pinv);
+      if (fwd_reduces(l)) ct<true>(x[k], x[k + h], w, p, pinv);
+      else ct<false>(x[k], x[k + h], w, p, pinv);
     }
   }
   __syncthreads();
@@ -272,14 +270,14 @@ __global__ __launch_bounds__(kThreads) void k_inv_cols(void* data, long long str
 // loads each coefficient once (the special IFFT output gathered in bit-reversed order, * 1/n,
 // * scale, rounded half away from zero: coefficient n < N/2 from the real part of slot brev(n),
 // n >= N/2 from the imaginary part of slot brev(n - N/2)), then for each of its limbs (lpb of them
-// from blockIdx.y lpb: a launch of few rows still fills the chip) takes the residue in [0, p) and
+// from blockIdx.y lpb: a launch of few rows still fills the chip) takes the centered residue and
 // runs stages 0..7 exactly as k_fwd_cols<kU64> does on stored residues, so the result is
 // bit-identical to rounding, storing every limb and transforming.  The residues of all limbs never
 // reach HBM.  Grid (16, limb chunks, rows).
 // Encoder cap: |coefficient| < 2^61, the reference's MAX_ENCODED_BITS
 // (llama3fhe/operators/attention/prefill/softmax.py:559).  A rounded coefficient is an exact double
-// (at and above 2^53 every double is an integer), and canon() reduces it exactly: q = floor(x / p)
-// is then below 2^12 and the residue x - q p (|.| < 2p) is the exact result of one FMA.
+// (at and above 2^53 every double is an integer), and reduce() centers it exactly: q = rint(x / p) is
+// below 2^30 and the residue x - q p the exact result of one FMA.
 constexpr double kEncodeCap = 2305843009213693952.0;  // 2^61
 
 __global__ __launch_bounds__(kThreads) void k_encode_cols(const double* __restrict__ vre,
@@ -316,7 +314,7 @@ __global__ __launch_bounds__(kThreads) void k_encode_cols(const double* __restri
     const double* __restrict__ tw = T.tw_fwd + (size_t)pi * kN;
     double x[16];
 #pragma unroll
-    for (int k = 0; k < 16; ++k) x[k] = canon(a[k], p, pinv);
+    for (int k = 0; k < 16; ++k) x[k] = reduce(a[k], p, pinv);
 #pragma unroll
     for (int l = 0; l < 4; ++l) {
       const int hh = 8 >> l;
@@ -324,8 +322,8 @@ __global__ __launch_bounds__(kThreads) void k_encode_cols(const double* __restri
       for (int k = 0; k < 16; ++k) {
         if (k & hh) continue;
         const double w = tw[(1 << l) + (k >> (4 - l))];
-        if (l & 1) ct<false>(x[k], x[k + hh], w, p, pinv);
-        else ct<true>(x[k], x[k + hh], w, p, pinv);
+        if (fwd_reduces(l)) ct<true>(x[k], x[k + hh], w, p, pinv);
+        else ct<false>(x[k], x[k + hh], w, p, pinv);
       }
     }
 #pragma unroll
@@ -341,8 +339,8 @@ __global__ __launch_bounds__(kThreads) void k_encode_cols(const double* __restri
       for (int k = 0; k < 16; ++k) {
         if (k & hh) continue;
         const double w = tw[(1 << l) + (j << (l - 4)) + (k >> (8 - l))];
-        if (l & 1) ct<false>(x[k], x[k + hh], w, p, pinv);
-        else ct<true>(x[k], x[k + hh], w, p, pinv);
+        if (fwd_reduces(l)) ct<true>(x[k], x[k + hh], w, p, pinv);
+        else ct<false>(x[k], x[k + hh], w, p, pinv);
       }
     }
     double* dl = d + (long long)list.off[e] * kN;
