@@ -83,6 +83,9 @@ SIGNATURES = {
     "hck_pack_diagonals": (_i, [_vp, _vp, _i, _i, _i, _i, _i, _i, _vp, _vp]),
     "hck_encode_workspace_bytes": (_sz, [_vp, _i]),
     "hck_encode": (_i, [_vp, _vp, _vp, _i, ctypes.c_double, _i, _ip, _vp, _i64, _vp, _sz, _vp, _vp]),
+    "hck_encode_cols": (_i, [_vp, _vp, _vp, _i, ctypes.c_double, _i, _ip, _vp, _i64, _vp, _sz, _vp, _vp]),
+    "hck_bsgs_mac_rows": (_i, [_vp, _i, _ip, _i, _i, _i, ctypes.POINTER(_vp), ctypes.POINTER(_vp), _i64, _vp, _i64,
+                               _vp, _vp]),
     "hck_tensor": (_i, [_vp, _i, _i, _vp, _vp, _i64, _vp, _vp, _i64, _vp, _vp, _vp, _i64, _vp]),
     "hck_relinearize_workspace_bytes": (_sz, [_vp, _i, _i]),
     "hck_relinearize": (_i, [_vp, _i, _i, _vp, _vp, _vp, _i64, _vp, _vp, _vp, _i64, _vp, _sz, _vp]),

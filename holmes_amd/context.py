@@ -941,7 +941,7 @@ class CKKSContext:
         return out
 
     def bsgs_mac(self, babies_c0, babies_c1, pts: torch.Tensor, limbs: int, giants: int,
-                 out: torch.Tensor | None = None, prime_idx=None) -> torch.Tensor:
+                 out: torch.Tensor | None = None, prime_idx=None, rows: bool = False) -> torch.Tensor:
         """Baby-step partial sums res[c][g][i] = sum_b pts[g*nb + b] * baby_b[i][c] (exact residues).
         babies_c0/c1: one [inputs][>=limbs][N] tensor per baby step (same batch stride); limb l
         uses prime prime_idx[l] (default: the first ``limbs`` Q primes)."""
@@ -966,12 +966,39 @@ class CKKSContext:
             out = self.empty(2, giants, ni, limbs, self.N)
         if tuple(out.shape) != (2, giants, ni, limbs, self.N) or not out.is_contiguous():
             raise ValueError("out must be a contiguous [2][giants][inputs][limbs][N] tensor")
-        nat.check(nat.lib().hck_bsgs_mac(self._h, limbs, nat.int_array(prime_idx), ni, nb, giants,
-                                         nat.ptr_array([t.data_ptr() for t in babies_c0]),
-                                         nat.ptr_array([t.data_ptr() for t in babies_c1]), stride,
-                                         pts.data_ptr(), _bstride(pts), out.data_ptr(),
-                                         _stream_ptr(self.device)), "hck_bsgs_mac")
+        fn, name = nat.lib().hck_bsgs_mac, "hck_bsgs_mac"
+        if rows:
+            fn, name = nat.lib().hck_bsgs_mac_rows, "hck_bsgs_mac_rows"
+        nat.check(fn(self._h, limbs, nat.int_array(prime_idx), ni, nb, giants,
+                     nat.ptr_array([t.data_ptr() for t in babies_c0]),
+                     nat.ptr_array([t.data_ptr() for t in babies_c1]), stride, pts.data_ptr(), _bstride(pts),
+                     out.data_ptr(), _stream_ptr(self.device)), name)
         return out
+
+    @property
+    def rows_mac(self) -> bool:
+        """Whether ``encode(..., row_pass=False)`` and ``bsgs_mac_rows`` exist here (FP64 kernels)."""
+
+        return max(self.primes) < 1 << 50
+
+    def rows_mac_pays(self, inputs: int, giants: int) -> bool:
+        """Whether ``bsgs_mac_rows`` beats encoding the plaintexts whole: its kernel takes one or two
+        inputs, 4 or 8 giants a workgroup, and transforms the empty slots' rows too.  Encode and
+        product over 8 babies x 3 limbs up to 32 x 17, times as fast: one input with 4 giants 1.11 to
+        1.47, 6 1.03 to 1.37, 9 1.03 to 1.46, 16 1.17 to 1.52 (1 giant 0.95 to 1.09, 3 0.95 to 1.40); two
+        with 6 1.00 to 1.27, 8 1.08 to 1.39, 16 1.05 to 1.36 (4 0.90 to 1.09, 9 0.91 to 1.15)."""
+
+        if not self.rows_mac or not 1 <= inputs <= 2 or giants < 4:
+            return False
+        slots = 4 if inputs == 1 else 8
+        return 4 * giants >= 3 * -(-giants // slots) * slots
+
+    def bsgs_mac_rows(self, babies_c0, babies_c1, pts: torch.Tensor, limbs: int, giants: int) -> torch.Tensor:
+        """``bsgs_mac`` of at most two inputs with plaintexts from ``encode(...,
+        row_pass=False)``: their row pass runs inside the product (hck_bsgs_mac_rows); the same residues
+        as encoding them whole."""
+
+        return self.bsgs_mac(babies_c0, babies_c1, pts, limbs, giants, rows=True)
 
     def pack_diagonals(self, weight: torch.Tensor, *, lanes: int, lane_shift: int, baby_steps: int,
                        giant_base: int, giant_count: int) -> torch.Tensor:
@@ -1015,7 +1042,8 @@ class CKKSContext:
         return v.to(torch.float64).repeat(1, reps).contiguous(), None
 
     def encode(self, values: torch.Tensor, scale: float, limbs: int, *, values_im: torch.Tensor | None = None,
-               prime_idx=None, out: torch.Tensor | None = None, flags: torch.Tensor | None = None) -> torch.Tensor:
+               prime_idx=None, out: torch.Tensor | None = None, flags: torch.Tensor | None = None,
+               row_pass: bool = True) -> torch.Tensor:
         """Encode slot rows [rows][N/2] (float64 on the device: real parts, optional imaginary parts)
         into NTT-domain residues [rows][limbs][N], limb l modulo prime prime_idx[l] (default: the
         first ``limbs`` Q primes; ``ext_prime_idx`` gives an extended-basis plaintext).
@@ -1023,7 +1051,10 @@ class CKKSContext:
         Overflow (a coefficient reaching 2^61) sets an int32 device flag per row.  Without
         ``flags`` they are read back here (one host sync) and raise; with a caller-owned
         ``flags`` tensor ([>= rows] int32, zeroed once) the flags accumulate there for one check
-        at the caller's next synchronisation point (``check_encode_flags``)."""
+        at the caller's next synchronisation point (``check_encode_flags``).
+
+        ``row_pass=False`` (contexts with ``rows_mac``) stops after the transform's column pass: the
+        words are doubles that only ``bsgs_mac_rows`` reads (hck_encode_cols)."""
 
         for v in (values,) + ((values_im,) if values_im is not None else ()):
             if v.dtype != torch.float64 or v.dim() != 2 or v.shape[1] != self.max_slots:
@@ -1049,10 +1080,11 @@ class CKKSContext:
             raise ValueError("flags must be a contiguous int32 tensor with one entry per row")
         L = nat.lib()
         ws = self.workspace(L.hck_encode_workspace_bytes(self._h, rows))
-        nat.check(L.hck_encode(self._h, values.data_ptr(), values_im.data_ptr() if values_im is not None else None,
-                               rows, float(scale), int(limbs), nat.int_array(prime_idx), out.data_ptr(),
-                               _bstride(out), ws.data_ptr(), ws.numel(), flags.data_ptr(),
-                               _stream_ptr(self.device)), "hck_encode")
+        fn = L.hck_encode if row_pass else L.hck_encode_cols
+        nat.check(fn(self._h, values.data_ptr(), values_im.data_ptr() if values_im is not None else None,
+                     rows, float(scale), int(limbs), nat.int_array(prime_idx), out.data_ptr(),
+                     _bstride(out), ws.data_ptr(), ws.numel(), flags.data_ptr(),
+                     _stream_ptr(self.device)), "hck_encode" if row_pass else "hck_encode_cols")
         if own:
             self.check_encode_flags(flags)
         return out

@@ -21,6 +21,7 @@
 #include "../../include/holmes_ckks.h"
 #include "internal.hpp"
 #include "mac_mx.hpp"
+#include "tile_layout.hpp"
 #include "wide.hpp"
 #include "modarith64.hpp"
 
@@ -153,6 +154,140 @@ __global__ __launch_bounds__(kMacThreads) void k_bsgs_mac(uint64_t* __restrict__
       for (int g = 0; g < kTG; ++g)
         if (g0 + g < G)
           res[c * cs + (long long)(g0 + g) * gs + (long long)(i0 + t) * is + ln] = d2u(canon(acc[t][c][g], p, pinv));
+  }
+}
+
+// ----------------------------------------------------------------- the MAC with the plaintexts' row pass
+// hck_bsgs_mac on plaintext rows that have had the transform's column pass only (hck_encode_cols): a
+// 256-word row of the 256 x 256 limb needs stages 8 .. 15, which stay inside it, so the workgroup that
+// multiplies the row transforms it.  Written and read back, a transformed plaintext costs 16 bytes of
+// HBM traffic per word against the 8 that this kernel reads; with one input the products take 17 FP64
+// operations per word and the row pass 36, so it stays near what HBM gives.  512 diagonals x 17 limbs,
+// encode and product: one input 4.35 -> 2.86 ms, two 4.59 -> 3.37 ms.  With more inputs the accumulators
+// do not fit the registers and the transform would be repeated.
+// Workgroup: one row of one limb, SL giants (slot s = t / 16 owns giant g0 + s, lane j = t % 16 of it words
+// j + 16 k before the exchange and 16 j + k after it), all babies in turn.  The row's twiddles are the
+// same for every plaintext: stages 8..11 in registers (uniform), 12..15 in LDS.  A baby's ciphertext row is
+// shared by the slots through LDS (two buffers, word 16 j + k at 17 k + j).  The next baby's words are in
+// flight while the current one is transformed.  |v| <= 5.5 p after the transform: |term| <= 2.6 p, the
+// sums are reduced every two babies.
+// SL: with one input 4 giants, a single wave (4, 8, 9, 16 giants x 32 babies: 0.84, 1.49, 1.82, 2.86 ms, 8
+// slots 1.03, 1.50, 2.07, 2.92, 16 slots 1.45, 1.88, 2.00, 2.84: fewer slots stand empty in the last
+// tile); with two inputs 8, since the two rows' words of a single wave spill (8 and 16 giants 1.73 and 3.37 ms,
+// 4 slots 1.88 and 3.72).
+constexpr int kMrRow = 272;
+constexpr int mr_slots(int inputs) { return inputs == 1 ? 4 : 8; }
+
+template <int NI>
+__global__ __launch_bounds__(16 * mr_slots(NI), 2) void k_mac_rows(
+    uint64_t* __restrict__ res, BabyPtrs babies, long long baby_stride, int nb, int ni, int G,
+    const double* __restrict__ pts, long long pt_stride, int limbs, MacPrimes mp, int tiles_g, DevTables T) {
+  constexpr int NC = 2 * NI;  // component c of input i: row 2 i + c
+  constexpr int SL = mr_slots(NI), TH = 16 * SL, XR = 16 / SL;  // row words per thread and component
+  __shared__ double R[SL * kMrRow], X[2][NC][kMrRow], W[15 * 16];
+  const int lin = blockIdx.x, xcd = lin % kXcds, q = lin / kXcds;
+  const int unit = (q / tiles_g) * kXcds + xcd, tile = q % tiles_g;  // limbs * 256 units, a multiple of 8
+  const int l = unit >> 8, row = unit & 255;
+  const int t = threadIdx.x, s = t >> 4, j = t & 15;
+  const int pi = mp.prime[l];
+  const double p = T.p[pi], pinv = T.pinv[pi];
+  const double* __restrict__ tw = T.tw_fwd + (size_t)pi * kN;
+  const long long ln = (long long)l * kN + row * 256;
+  const int g = min(tile * SL + s, G - 1);  // clamped slots are never stored
+  const double* prow = pts + (long long)g * nb * pt_stride + ln + j;
+  double lo[15];
+#pragma unroll
+  for (int i = 0; i < 15; ++i) {  // stage 8 + log2(i + 1): entry i + 1 of the row's heap
+    const int st = i >= 7 ? 3 : i >= 3 ? 2 : i >= 1 ? 1 : 0;
+    lo[i] = tw[(1 << (8 + st)) + (row << st) + (i + 1 - (1 << st))];
+  }
+  for (int w = t; w < 240; w += TH) {
+    const int i = w >> 4, st = i >= 7 ? 3 : i >= 3 ? 2 : i >= 1 ? 1 : 0;
+    W[w] = tw[(1 << (12 + st)) + (row << (4 + st)) + (j << st) + (i + 1 - (1 << st))];
+  }
+  double acc[NC][16], v[16], vn[16];
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int k = 0; k < 16; ++k) acc[c][k] = 0.0;
+  uint64_t xw[NC][XR];
+  auto load = [&](double (&d)[16], int b) {
+#pragma unroll
+    for (int k = 0; k < 16; ++k) d[k] = prow[(long long)b * pt_stride + 16 * k];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const int i = c >> 1;
+      const uint64_t* base = (c & 1) ? babies.c1[b] : babies.c0[b];
+#pragma unroll
+      for (int r = 0; r < XR; ++r) xw[c][r] = base[(i < ni ? i : 0) * baby_stride + ln + t + r * TH];
+    }
+  };
+  auto put = [&](int buf) {
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int r = 0; r < XR; ++r) X[buf][c][17 * (t & 15) + (t >> 4) + r * SL] = u2d(xw[c][r]);
+  };
+  double* Rs = R + s * kMrRow;
+  load(v, 0);
+  put(0);
+  __syncthreads();
+  for (int b = 0; b < nb; ++b) {
+    load(vn, b + 1 < nb ? b + 1 : b);  // the last step reloads its own words, unused
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int st = 0; st < 4; ++st) {
+      const int h = 8 >> st;
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        if (k & h) continue;
+        const double m = mulv(v[k + h], lo[(1 << st) - 1 + (k >> (4 - st))], p, pinv);
+        const double a = fwd_reduces(8 + st) ? reduce(v[k], p, pinv) : v[k];
+        v[k] = a + m;
+        v[k + h] = a - m;
+      }
+    }
+    col_a_to_b(v, Rs, j);
+#pragma unroll
+    for (int st = 0; st < 4; ++st) {
+      const int h = 8 >> st;
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        if (k & h) continue;
+        const double m = mulv(v[k + h], W[((1 << st) - 1 + (k >> (4 - st))) * 16 + j], p, pinv);
+        const double a = fwd_reduces(12 + st) ? reduce(v[k], p, pinv) : v[k];
+        v[k] = a + m;
+        v[k + h] = a - m;
+      }
+    }
+    const double(&xb)[NC][kMrRow] = X[b & 1];
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int k = 0; k < 16; ++k) acc[c][k] += mulv(v[k], xb[c][17 * k + j], p, pinv);
+    if (b & 1) {
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int k = 0; k < 16; ++k) acc[c][k] = reduce(acc[c][k], p, pinv);
+    }
+    put((b + 1) & 1);  // read last in the step before this one
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 16; ++k) v[k] = vn[k];
+  }
+  const long long is = (long long)limbs * kN, gs = (long long)ni * is, cs = (long long)G * gs;
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const int i = c >> 1;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) acc[c][k] = canon(acc[c][k], p, pinv);
+    col_b_to_a(acc[c], Rs, j);
+    if (i < ni && tile * SL + s < G) {
+      uint64_t* o = res + (c & 1) * cs + (long long)g * gs + (long long)i * is + ln + j;
+#pragma unroll
+      for (int k = 0; k < 16; ++k) o[16 * k] = d2u(acc[c][k]);
+    }
   }
 }
 
@@ -332,6 +467,35 @@ extern "C" int hck_bsgs_mac(const hck_context* ctx, int limbs, const int* prime_
   k<<<dim3((unsigned)blocks), hck::kMacThreads, 0, (hipStream_t)stream>>>(
       res, bp, baby_stride, babies, inputs, giants, pts, pt_stride, limbs, mp, units_per_limb, tiles_i, tiles_g,
       total_units, ctx->dev);
+  HCK_CHECK_LAUNCH();
+  return HCK_OK;
+}
+
+extern "C" int hck_bsgs_mac_rows(const hck_context* ctx, int limbs, const int* prime_idx, int inputs, int babies,
+                                 int giants, const uint64_t* const* baby_c0, const uint64_t* const* baby_c1,
+                                 int64_t baby_stride, const double* pts, int64_t pt_stride, uint64_t* res,
+                                 void* stream) {
+  if (!ctx || !prime_idx || !baby_c0 || !baby_c1 || !pts || !res) return HCK_ERR_ARG;
+  if (limbs < 1 || limbs > hck::kMaxPrimes || inputs < 1 || babies < 1 || babies > hck::kMaxBabies || giants < 1)
+    return HCK_ERR_ARG;
+  if (ctx->wide || inputs > HCK_MAC_ROWS_INPUTS) return HCK_ERR_UNSUPPORTED;
+  hck::MacPrimes mp{};
+  for (int l = 0; l < limbs; ++l) {
+    if (prime_idx[l] < 0 || prime_idx[l] >= ctx->np) return HCK_ERR_ARG;
+    mp.prime[l] = (uint8_t)prime_idx[l];
+  }
+  hck::BabyPtrs bp{};
+  for (int b = 0; b < babies; ++b) {
+    if (!baby_c0[b] || !baby_c1[b]) return HCK_ERR_ARG;
+    bp.c0[b] = baby_c0[b];
+    bp.c1[b] = baby_c1[b];
+  }
+  const int slots = hck::mr_slots(inputs), tiles_g = (giants + slots - 1) / slots;
+  const long long blocks = (long long)limbs * 256 * tiles_g;
+  if (blocks > 0x7fffffffLL) return HCK_ERR_ARG;
+  auto k = inputs == 1 ? hck::k_mac_rows<1> : hck::k_mac_rows<2>;
+  k<<<dim3((unsigned)blocks), 16 * slots, 0, (hipStream_t)stream>>>(
+      res, bp, baby_stride, babies, inputs, giants, pts, pt_stride, limbs, mp, tiles_g, ctx->dev);
   HCK_CHECK_LAUNCH();
   return HCK_OK;
 }

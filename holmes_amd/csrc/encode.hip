@@ -200,9 +200,10 @@ extern "C" size_t hck_encode_workspace_bytes(const hck_context* ctx, int rows) {
   return (size_t)rows * hck::kSlots * 2 * sizeof(double) + (size_t)rows * sizeof(int) + 256;
 }
 
-extern "C" int hck_encode(const hck_context* ctx, const double* values, const double* values_im, int rows,
-                          double scale, int limbs, const int* prime_idx, uint64_t* out, int64_t out_row_stride,
-                          void* workspace, size_t workspace_bytes, int* overflow_flags, void* stream) {
+namespace {
+int encode_rows(const hck_context* ctx, const double* values, const double* values_im, int rows, double scale, int limbs,
+                const int* prime_idx, uint64_t* out, int64_t out_row_stride, void* workspace, size_t workspace_bytes,
+                int* overflow_flags, void* stream, bool row_pass) {
   if (!ctx || !values || !out || !prime_idx || !overflow_flags || rows < 0 || rows > 65535) return HCK_ERR_ARG;
   if (limbs < 1 || limbs > hck::kMaxPrimes || !(scale > 0.0)) return HCK_ERR_ARG;
   if (rows == 0) return HCK_OK;
@@ -223,7 +224,23 @@ extern "C" int hck_encode(const hck_context* ctx, const double* values, const do
   hck::k_sifft_rows<<<dim3(256 / 32, rows), 256, 0, s>>>(vre, vim, ctx->d_enc_twr, ctx->d_enc_twi);
   HCK_CHECK_LAUNCH();
   // rounding, residues and the NTT's column pass in one kernel, then the row pass
-  return hck::launch_encode_ntt(ctx, vre, vim, scale, out, out_row_stride, rows, overflow_flags, L, s);
+  return hck::launch_encode_ntt(ctx, vre, vim, scale, out, out_row_stride, rows, overflow_flags, L, s, row_pass);
+}
+}  // namespace
+
+extern "C" int hck_encode(const hck_context* ctx, const double* values, const double* values_im, int rows,
+                          double scale, int limbs, const int* prime_idx, uint64_t* out, int64_t out_row_stride,
+                          void* workspace, size_t workspace_bytes, int* overflow_flags, void* stream) {
+  return encode_rows(ctx, values, values_im, rows, scale, limbs, prime_idx, out, out_row_stride, workspace,
+                     workspace_bytes, overflow_flags, stream, true);
+}
+
+extern "C" int hck_encode_cols(const hck_context* ctx, const double* values, const double* values_im, int rows,
+                               double scale, int limbs, const int* prime_idx, double* out, int64_t out_row_stride,
+                               void* workspace, size_t workspace_bytes, int* overflow_flags, void* stream) {
+  if (ctx && ctx->wide) return HCK_ERR_UNSUPPORTED;
+  return encode_rows(ctx, values, values_im, rows, scale, limbs, prime_idx, (uint64_t*)out, out_row_stride, workspace,
+                     workspace_bytes, overflow_flags, stream, false);
 }
 
 // The reference's encode sidecar entry point with its argument list (bench/cmp/kernels/

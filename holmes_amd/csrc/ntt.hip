@@ -373,8 +373,9 @@ int launch_ntt_fwd(const hck_context* c, const void* src, Fmt in, void* dst, Fmt
 }
 
 int launch_encode_ntt(const hck_context* c, const double* vre, const double* vim, double scale, uint64_t* out,
-                      long long out_stride, int rows, int* overflow, const LimbList& list, hipStream_t s) {
-  if (c->wide) return wide_encode_ntt(c, vre, vim, scale, out, out_stride, rows, overflow, list, s);
+                      long long out_stride, int rows, int* overflow, const LimbList& list, hipStream_t s, bool row_pass) {
+  if (c->wide)
+    return row_pass ? wide_encode_ntt(c, vre, vim, scale, out, out_stride, rows, overflow, list, s) : HCK_ERR_UNSUPPORTED;
   if (list.n <= 0 || rows <= 0) return HCK_OK;
   if (list.n > kMaxList || rows > 65535) return HCK_ERR_ARG;
   // limbs split over blockIdx.y so that a launch of few rows still fills the chip (each block rounds
@@ -382,7 +383,7 @@ int launch_encode_ntt(const hck_context* c, const double* vre, const double* vim
   const int lpb = encode_limbs_per_block(list.n, rows);
   k_encode_cols<<<dim3(16, (list.n + lpb - 1) / lpb, rows), kThreads, 0, s>>>(vre, vim, scale, (double*)out,
                                                                             out_stride, list, lpb, overflow, c->dev);
-  k_fwd_rows<kU64><<<dim3(16, list.n, rows), kThreads, 0, s>>>(out, out_stride, list, c->dev);
+  if (row_pass) k_fwd_rows<kU64><<<dim3(16, list.n, rows), kThreads, 0, s>>>(out, out_stride, list, c->dev);
   HCK_CHECK_LAUNCH();
   return HCK_OK;
 }

@@ -83,6 +83,13 @@ class Plaintext:
         self.cv = []
 
 
+class ColumnPlaintext(Plaintext):
+    """Plaintext rows that have had the transform's column pass only (``CKKSContext.encode(...,
+    row_pass=False)``): ``hoisted_mac_sum`` finishes them inside its multiply-accumulate."""
+
+    __slots__ = ()
+
+
 def generate_client_context(spec: CKKSContextSpec, device: str = "cuda"):
     """Build the context (device tables) and the client (secret key) with the relinearisation key;
     generate the requested rotation keys when ``spec.auto_load_keys``.  Returns
@@ -628,8 +635,9 @@ def hoisted_mac_sum(ct: Cipher, baby_offsets, plaintexts: Plaintext, giant_offse
     pt_state = plaintexts.state if isinstance(plaintexts, Plaintext) else None
     if pts.shape[0] != nb * G:
         raise ValueError(f"expected {nb * G} plaintext rows, got {pts.shape[0]}")
-    part = ctx.bsgs_mac([_view(b.cv[0], limbs) for b in babies], [_view(b.cv[1], limbs) for b in babies],
-                        pts, limbs, G)  # [2][G][B][limbs][N]
+    mac = ctx.bsgs_mac_rows if isinstance(plaintexts, ColumnPlaintext) else ctx.bsgs_mac
+    part = mac([_view(b.cv[0], limbs) for b in babies], [_view(b.cv[1], limbs) for b in babies],
+               pts, limbs, G)  # [2][G][B][limbs][N]
     idx = ctx.q_prime_idx(limbs)
     if strategy == "ext_double_hoist" and G > 1:
         ext0 = _lift_ext(part[0, 0], limbs, ctx)

@@ -245,9 +245,10 @@ class LinearWeight:
         return self._wi is not None
 
     def plaintext(self, plan: LinearPlan, chunk: LinearChunk, *, limbs: int, scale: float,
-                  flags: torch.Tensor | None = None) -> torch.Tensor:
+                  flags: torch.Tensor | None = None, row_pass: bool = True) -> torch.Tensor:
         """Encoded diagonals [giant_count * baby_steps][limbs][N] of ``chunk`` (NTT domain).
-        ``flags`` (int32, one per row) defers the overflow check to the caller."""
+        ``flags`` (int32, one per row) defers the overflow check to the caller; ``row_pass=False``
+        leaves the transform's row pass to the multiply-accumulate (``fhe.ColumnPlaintext``)."""
 
         if self._closed:
             raise RuntimeError("linear weight is closed")
@@ -259,8 +260,8 @@ class LinearWeight:
                                       giant_count=chunk.giant_count)
 
         if self._wi is None:
-            return ctx.encode_real(rows(self._w), scale, limbs, flags=flags)
-        return ctx.encode(rows(self._w), scale, limbs, values_im=rows(self._wi), flags=flags)
+            return ctx.encode(rows(self._w), scale, limbs, flags=flags, row_pass=row_pass)
+        return ctx.encode(rows(self._w), scale, limbs, values_im=rows(self._wi), flags=flags, row_pass=row_pass)
 
     def close(self) -> None:
         self._w = None
@@ -364,8 +365,11 @@ class LinearOperator:
         flags = torch.zeros(int(plan.max_plaintext_rows), dtype=torch.int32, device=x0.device)
         pt_state = CipherState(cur_limbs=limbs, scale_degree=1, scaling_factor=wscale)
         for chunk in chunks:
-            pts = fhe.Plaintext(weight.plaintext(plan, chunk, limbs=limbs, scale=wscale, flags=flags), pt_state,
-                                slots=xc.slots)
+            args = dict(limbs=limbs, scale=wscale, flags=flags)
+            kind = fhe.Plaintext
+            if type(weight) is LinearWeight and ctx.rows_mac_pays(int(x0.shape[0]), int(chunk.giant_count)):
+                kind, args["row_pass"] = fhe.ColumnPlaintext, False
+            pts = kind(weight.plaintext(plan, chunk, **args), pt_state, slots=xc.slots)
             res = fhe.hoisted_mac_sum(xc, plan.baby_offsets, pts, plan.giant_offset, int(chunk.giant_count), ctx,
                                       strategy=strategy, baby_anchor_step=int(plan.baby_anchor_step),
                                       baby_rotations=babies)

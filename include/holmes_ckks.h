@@ -275,6 +275,14 @@ int hck_poly_from_signed(const hck_context* ctx, const int64_t* in, uint64_t* ou
 int hck_bsgs_mac(const hck_context* ctx, int limbs, const int* prime_idx, int inputs, int babies, int giants,
                  const uint64_t* const* baby_c0, const uint64_t* const* baby_c1, int64_t baby_stride,
                  const uint64_t* pts, int64_t pt_stride, uint64_t* res, void* stream);
+/* hck_bsgs_mac on plaintext rows that hck_encode_cols wrote: the transform's row pass runs inside the
+ * product, so the transformed plaintexts are neither written nor read back.  The same residues as
+ * hck_encode followed by hck_bsgs_mac.  At most HCK_MAC_ROWS_INPUTS inputs; FP64 contexts only
+ * (HCK_ERR_UNSUPPORTED otherwise).  A plaintext serves one call: the row pass is paid per call. */
+#define HCK_MAC_ROWS_INPUTS 2
+int hck_bsgs_mac_rows(const hck_context* ctx, int limbs, const int* prime_idx, int inputs, int babies, int giants,
+                      const uint64_t* const* baby_c0, const uint64_t* const* baby_c1, int64_t baby_stride,
+                      const double* pts, int64_t pt_stride, uint64_t* res, void* stream);
 
 /* The reference sidecar's multi-input MAC, argument for argument (bench/cmp/kernels/holmes_mac.cu:359-402,
  * bound by ctypes at bench/cmp/holmes_multi_mac.py:49, called at :138):
@@ -306,6 +314,12 @@ size_t hck_encode_workspace_bytes(const hck_context* ctx, int rows);
 int hck_encode(const hck_context* ctx, const double* values, const double* values_im, int rows, double scale,
                int limbs, const int* prime_idx, uint64_t* out, int64_t out_row_stride, void* workspace,
                size_t workspace_bytes, int* overflow_flags, void* stream);
+/* hck_encode without the transform's row pass (stages 8 .. 15): `out` holds [rows][limbs][N] doubles, the
+ * rows that hck_bsgs_mac_rows multiplies.  Same arguments, workspace and flags.  FP64 contexts only
+ * (HCK_ERR_UNSUPPORTED with a prime at or above 2^50). */
+int hck_encode_cols(const hck_context* ctx, const double* values, const double* values_im, int rows, double scale,
+                    int limbs, const int* prime_idx, double* out, int64_t out_row_stride, void* workspace,
+                    size_t workspace_bytes, int* overflow_flags, void* stream);
 
 /* The reference's encode sidecar, holmes_encode_stage2, with its argument list and return
  * convention (bench/cmp/kernels/holmes_encode.cu:240-285; bound with the argtypes of

@@ -61,3 +61,30 @@ def test_vector_tiles(env, ni, nb, G, limbs):
 def test_rows_that_are_not_16_byte_aligned(env):
     """A shape of the matrix-core kernel whose plaintexts start at an odd word."""
     _check(env, 8, 16, 16, 1, offset=1)
+
+
+@pytest.mark.parametrize("ni,nb,G,limbs", [(1, 16, 32, 2), (1, 1, 1, 1), (2, 5, 17, 1), (2, 16, 7, 1), (1, 64, 5, 1)])
+def test_row_pass_inside_the_product(env, ni, nb, G, limbs):
+    """Plaintexts with the column pass only, finished inside the product, against encoding them whole
+    (bit-exact against the oracle in test_gpu_bsgs); the wide path refuses them."""
+    from holmes_amd import _native as nat
+
+    ctx, _ = env
+    gen = torch.Generator(device="cuda").manual_seed(nb * 100 + G)
+    re, im = (torch.randn(G * nb, ctx.max_slots, dtype=torch.float64, device="cuda", generator=gen) for _ in range(2))
+    scale = float(ctx.rescale_divisor_at(2))
+    if not ctx.rows_mac:
+        with pytest.raises(nat.NativeError):
+            ctx.encode(re, scale, limbs, values_im=im, row_pass=False)
+        return
+    q = torch.tensor([int(p) for p in ctx.primes[:limbs]], dtype=torch.int64, device="cuda")[:, None]
+    x = torch.randint(0, 1 << 62, (nb, 2, ni, limbs, ctx.N), dtype=torch.int64, device="cuda", generator=gen)
+    x.remainder_(q)
+    x[..., :2] = q - 1
+    x = x.view(torch.uint64)
+    b0, b1 = [x[b, 0] for b in range(nb)], [x[b, 1] for b in range(nb)]
+    want = ctx.bsgs_mac(b0, b1, ctx.encode(re, scale, limbs, values_im=im), limbs, G)
+    got = ctx.bsgs_mac_rows(b0, b1, ctx.encode(re, scale, limbs, values_im=im, row_pass=False), limbs, G)
+    assert torch.equal(got.view(torch.int64), want.view(torch.int64))
+    with pytest.raises(nat.NativeError):
+        ctx.bsgs_mac_rows([ctx.zeros(3, 1, ctx.N)], [ctx.zeros(3, 1, ctx.N)], ctx.zeros(1, 1, ctx.N), 1, 1)
