@@ -90,11 +90,9 @@ constexpr bool fwd_reduces(int l) { return l == 3 || l == 6 || l == 9 || l == 11
 // toolchain does not send negative ties away from zero.  trunc, one exact subtraction and two
 // comparisons: no product to contract, so the result is the same in every translation unit.
 __device__ __forceinline__ double round_away(double x) {
-  double r = __builtin_trunc(x);
+  const double r = __builtin_trunc(x);
   const double d = x - r;  // exact
-  if (d >= 0.5) r += 1.0;
-  else if (d <= -0.5) r -= 1.0;
-  return r;
+  return r + __builtin_copysign(__builtin_fabs(d) >= 0.5 ? 1.0 : 0.0, x);
 }
 
 }  // namespace hck

@@ -280,6 +280,33 @@ __global__ __launch_bounds__(kThreads) void k_inv_cols(void* data, long long str
 // below 2^30 and the residue x - q p the exact result of one FMA.
 constexpr double kEncodeCap = 2305843009213693952.0;  // 2^61
 
+// One limb's constants.  The tables and the kernel's arguments are read only while it runs: the uniform
+// ones go through constant-address pointers, i.e. the scalar cache, and the lane's stage 4..7 twiddles
+// are issued as one batch before the previous limb's stores (loads and stores retire in order).  Read
+// where the stages use them, the constants cost eight dependent rounds of loads a limb, the first behind
+// the previous limb's stores, and the sixteen gathers, each rounded in branches, sixteen more: 96 complex
+// rows x 13 limbs 616 -> 579 us in all.  (Four waves per SIMD spill: 761 us.)
+template <typename E>
+using ConstPtr = const __attribute__((address_space(4))) E*;
+static_assert(offsetof(LimbList, off) % 4 == 0 && offsetof(LimbList, prime) % 4 == 0, "read by words");
+struct EncTw {
+  double p, pinv, lo[15], hi[15];
+  unsigned off;
+  __device__ __forceinline__ void load(const LimbList& list, int e, int j, const DevTables& T) {
+    const unsigned pi = (((ConstPtr<unsigned>)list.prime)[e >> 2] >> (8 * (e & 3))) & 255;
+    off = (((ConstPtr<unsigned>)list.off)[e >> 1] >> (16 * (e & 1))) & 65535;
+    p = ((ConstPtr<double>)T.p)[pi];
+    pinv = ((ConstPtr<double>)T.pinv)[pi];
+    const double* tw = T.tw_fwd + (size_t)pi * kN;
+#pragma unroll
+    for (int i = 0; i < 15; ++i) lo[i] = ((ConstPtr<double>)tw)[i + 1];
+#pragma unroll
+    for (int l = 4; l < 8; ++l)
+#pragma unroll
+      for (int i = 0; i < 1 << (l - 4); ++i) hi[(1 << (l - 4)) - 1 + i] = tw[(1 << l) + (unsigned)((j << (l - 4)) + i)];
+  }
+};
+
 __global__ __launch_bounds__(kThreads) void k_encode_cols(const double* __restrict__ vre,
                                                           const double* __restrict__ vim, double scale,
                                                           double* __restrict__ out, long long out_stride,
@@ -300,18 +327,23 @@ __global__ __launch_bounds__(kThreads) void k_encode_cols(const double* __restri
       const int n = (j + 16 * k) * 256 + c;
       const int h = n >= kN / 2;
       const int slot = (int)(__brev((unsigned)(n - h * (kN / 2))) >> (32 - (kLogN - 1)));
-      const double w = (h ? im : re)[slot] * inv_n;
-      a[k] = round_away(w * scale);
+      a[k] = (h ? im : re)[slot];
+    }
+    __builtin_amdgcn_sched_barrier(0);  // all sixteen gathers in flight
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      a[k] = round_away(a[k] * inv_n * scale);
       big |= fabs(a[k]) >= kEncodeCap;
     }
   }
   if (big) overflow[row] = 1;
   double* d = out + row * out_stride;
   const int e_end = min(list.n, ((int)blockIdx.y + 1) * lpb);  // this block: limbs [blockIdx.y lpb, e_end)
-  for (int e = (int)blockIdx.y * lpb; e < e_end; ++e) {
-    const int pi = list.prime[e];
-    const double p = T.p[pi], pinv = T.pinv[pi];
-    const double* __restrict__ tw = T.tw_fwd + (size_t)pi * kN;
+  int e = (int)blockIdx.y * lpb;
+  EncTw w;
+  w.load(list, e, j, T);
+  for (; e < e_end; ++e) {
+    const double p = w.p, pinv = w.pinv;
     double x[16];
 #pragma unroll
     for (int k = 0; k < 16; ++k) x[k] = reduce(a[k], p, pinv);
@@ -321,9 +353,9 @@ __global__ __launch_bounds__(kThreads) void k_encode_cols(const double* __restri
 #pragma unroll
       for (int k = 0; k < 16; ++k) {
         if (k & hh) continue;
-        const double w = tw[(1 << l) + (k >> (4 - l))];
-        if (fwd_reduces(l)) ct<true>(x[k], x[k + hh], w, p, pinv);
-        else ct<false>(x[k], x[k + hh], w, p, pinv);
+        const double wk = w.lo[(1 << l) - 1 + (k >> (4 - l))];
+        if (fwd_reduces(l)) ct<true>(x[k], x[k + hh], wk, p, pinv);
+        else ct<false>(x[k], x[k + hh], wk, p, pinv);
       }
     }
 #pragma unroll
@@ -338,14 +370,16 @@ __global__ __launch_bounds__(kThreads) void k_encode_cols(const double* __restri
 #pragma unroll
       for (int k = 0; k < 16; ++k) {
         if (k & hh) continue;
-        const double w = tw[(1 << l) + (j << (l - 4)) + (k >> (8 - l))];
-        if (fwd_reduces(l)) ct<true>(x[k], x[k + hh], w, p, pinv);
-        else ct<false>(x[k], x[k + hh], w, p, pinv);
+        const double wk = w.hi[(1 << (l - 4)) - 1 + (k >> (8 - l))];
+        if (fwd_reduces(l)) ct<true>(x[k], x[k + hh], wk, p, pinv);
+        else ct<false>(x[k], x[k + hh], wk, p, pinv);
       }
     }
-    double* dl = d + (long long)list.off[e] * kN;
+    double* dl = d + (size_t)w.off * kN;
+    if (e + 1 < e_end) w.load(list, e + 1, j, T);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int k = 0; k < 16; ++k) dl[(long long)(16 * j + k) * 256 + c] = x[k];
+    for (int k = 0; k < 16; ++k) (dl + k * 256)[(unsigned)(16 * j * 256 + c)] = x[k];
   }
 }
 
