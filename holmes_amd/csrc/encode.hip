@@ -40,18 +40,33 @@ __device__ __forceinline__ void sbf(Cx& u, Cx& v, double wr, double wi) {
   v.im = dr * wi + di * wr;
 }
 
+// Thread: one slot of one giant, kPackBabies baby steps.  Neighbouring baby steps read neighbouring words
+// of a weight row, so a thread's reads share cache lines and its index arithmetic (64-bit remainders) is
+// paid once: 512 diagonals of a 4096 x 4096 weight 133 -> 94 us (one thread per word before).
+constexpr int kPackBabies = 8;
+
 __global__ __launch_bounds__(256) void k_pack_diagonals(const double* __restrict__ W, int D, int lanes,
-                                                        int lane_shift, int baby_steps, int giant_base,
+                                                        int lane_shift, int baby_steps, int chunks, int giant_base,
                                                         double* __restrict__ out) {
-  const int s = blockIdx.x * 256 + threadIdx.x;
-  const int row = blockIdx.y;
-  const int gr = row / baby_steps, b = row % baby_steps;
-  const long long g = giant_base + gr;
-  const long long f = s / lanes, lane = s % lanes;
-  long long o = (f - g * baby_steps) % D;
+  const unsigned s = blockIdx.x * 256 + threadIdx.x;
+  const int gr = blockIdx.y / chunks, b0 = (blockIdx.y % chunks) * kPackBabies;
+  const int n = min(kPackBabies, baby_steps - b0);
+  const long long g = (long long)giant_base + gr;
+  const unsigned f = s / (unsigned)lanes, lane = s % (unsigned)lanes;
+  long long o = ((long long)f - g * baby_steps) % D;
   if (o < 0) o += D;
-  const long long in = (f + b + (long long)lane_shift * lane) % D;
-  out[(long long)row * kSlots + s] = W[o * D + in];
+  long long in = ((long long)f + b0 + (long long)lane_shift * lane) % D;
+  const double* w = W + o * D;
+  double v[kPackBabies];
+#pragma unroll
+  for (int k = 0; k < kPackBabies; ++k) {
+    v[k] = w[in];  // past the last baby step: still inside the row
+    in = in + 1 == D ? 0 : in + 1;
+  }
+  double* q = out + ((long long)gr * baby_steps + b0) * kSlots + s;
+#pragma unroll
+  for (int k = 0; k < kPackBabies; ++k)
+    if (k < n) q[(long long)k * kSlots] = v[k];
 }
 
 // Column pass: block = 16 columns x 256 rows of one row-vector; thread (cl, j) holds rows j + 16k
@@ -189,8 +204,9 @@ extern "C" int hck_pack_diagonals(const hck_context* ctx, const double* weight, 
     return HCK_ERR_ARG;
   const long long rows = (long long)giant_count * baby_steps;
   if (rows > 65535) return HCK_ERR_ARG;
-  hck::k_pack_diagonals<<<dim3(hck::kSlots / 256, (unsigned)rows), 256, 0, (hipStream_t)stream>>>(
-      weight, dimension, lanes, lane_shift, baby_steps, giant_base, out);
+  const int chunks = (baby_steps + hck::kPackBabies - 1) / hck::kPackBabies;  // giant_count * chunks <= rows
+  hck::k_pack_diagonals<<<dim3(hck::kSlots / 256, (unsigned)(giant_count * chunks)), 256, 0, (hipStream_t)stream>>>(
+      weight, dimension, lanes, lane_shift, baby_steps, chunks, giant_base, out);
   HCK_CHECK_LAUNCH();
   return HCK_OK;
 }

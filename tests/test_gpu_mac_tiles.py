@@ -88,3 +88,14 @@ def test_row_pass_inside_the_product(env, ni, nb, G, limbs):
     assert torch.equal(got.view(torch.int64), want.view(torch.int64))
     with pytest.raises(nat.NativeError):
         ctx.bsgs_mac_rows([ctx.zeros(3, 1, ctx.N)], [ctx.zeros(3, 1, ctx.N)], ctx.zeros(1, 1, ctx.N), 1, 1)
+
+
+@pytest.mark.parametrize("D,lanes,shift,B,base,G", [(96, 4, 0, 1, 0, 3), (96, 8, 5, 7, 2, 2), (64, 1, 0, 9, 1, 2),
+                                                    (1, 2, 3, 17, 0, 1)])
+def test_packed_baby_chunks(env, D, lanes, shift, B, base, G):
+    """The packer's groups of 8 baby steps: alone, one short, one more, rows shorter than a group."""
+    ctx, _ = env
+    W = np.random.default_rng(B).standard_normal((D, D))
+    got = ctx.pack_diagonals(torch.from_numpy(W).cuda(), lanes=lanes, lane_shift=shift, baby_steps=B,
+                             giant_base=base, giant_count=G).cpu().numpy()
+    assert np.array_equal(got, O.pack_diagonals(W, lanes, shift, B, base, G, ctx.max_slots))
