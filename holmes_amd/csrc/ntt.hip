@@ -280,21 +280,33 @@ __global__ __launch_bounds__(kThreads) void k_inv_cols(void* data, long long str
 // below 2^30 and the residue x - q p the exact result of one FMA.
 constexpr double kEncodeCap = 2305843009213693952.0;  // 2^61
 
-// One limb's constants.  The tables and the kernel's arguments are read only while it runs: the uniform
-// ones go through constant-address pointers, i.e. the scalar cache, and the lane's stage 4..7 twiddles
-// are issued as one batch before the previous limb's stores (loads and stores retire in order).  Read
-// where the stages use them, the constants cost eight dependent rounds of loads a limb, the first behind
-// the previous limb's stores, and the sixteen gathers, each rounded in branches, sixteen more: 96 complex
-// rows x 13 limbs 616 -> 579 us in all.  (Four waves per SIMD spill: 761 us.)
+// One limb's constants.  The tables are read only while the kernel runs: the uniform ones go through
+// constant-address pointers, i.e. the scalar cache, and the lane's stage 4..7 twiddles are issued as one
+// batch before the previous limb's stores (loads and stores retire in order).  Read where the stages use
+// them, the constants cost eight dependent rounds of loads a limb, the first behind the previous limb's
+// stores, and the sixteen gathers, each rounded in branches, sixteen more: 96 complex rows x 13 limbs
+// 616 -> 579 us in all.  (Four waves per SIMD spill: 761 us.)
 template <typename E>
 using ConstPtr = const __attribute__((address_space(4))) E*;
-static_assert(offsetof(LimbList, off) % 4 == 0 && offsetof(LimbList, prime) % 4 == 0, "read by words");
+
+// Entry i of an array of 8- or 16-bit entries as a field of the aligned 32-bit word that holds it: a scalar
+// load of the argument segment, where an entry of its own would be a vector load.
+template <typename E>
+__device__ __forceinline__ unsigned packed_entry(const E* a, unsigned i) {
+  constexpr unsigned kPer = 4 / sizeof(E);
+  uint32_t w;
+  __builtin_memcpy(&w, __builtin_assume_aligned(a + i / kPer * kPer, 4), 4);
+  return (w >> (8 * sizeof(E) * (i % kPer))) & ((1u << (8 * sizeof(E))) - 1);
+}
+static_assert(alignof(LimbList) % 4 == 0 && offsetof(LimbList, off) % 4 == 0 && offsetof(LimbList, prime) % 4 == 0,
+              "entries are read by words");
+
 struct EncTw {
   double p, pinv, lo[15], hi[15];
   unsigned off;
   __device__ __forceinline__ void load(const LimbList& list, int e, int j, const DevTables& T) {
-    const unsigned pi = (((ConstPtr<unsigned>)list.prime)[e >> 2] >> (8 * (e & 3))) & 255;
-    off = (((ConstPtr<unsigned>)list.off)[e >> 1] >> (16 * (e & 1))) & 65535;
+    const unsigned pi = packed_entry(list.prime, e);
+    off = packed_entry(list.off, e);
     p = ((ConstPtr<double>)T.p)[pi];
     pinv = ((ConstPtr<double>)T.pinv)[pi];
     const double* tw = T.tw_fwd + (size_t)pi * kN;
