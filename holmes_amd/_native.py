@@ -15,6 +15,7 @@ HCK_ERR_ARG = -1
 HCK_ERR_WORKSPACE = -5
 HCK_ERR_SCRATCH = -6
 HCK_NOALLOC_SCRATCH_BYTES = 128 << 20   # include/holmes_ckks.h: the array behind hck_rotate_noalloc
+HCK_MAC_ROWS_INPUTS = 2                 # include/holmes_ckks.h: inputs of hck_bsgs_mac_rows
 
 HCK_OP_ADD = 0
 HCK_OP_SUB = 1

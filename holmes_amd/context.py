@@ -337,9 +337,9 @@ class CKKSContext:
 
     # ------------------------------------------------------------------ kernels
     @staticmethod
-    def _check_poly(t: torch.Tensor, limbs: int, n: int) -> None:
-        if t.dtype != torch.uint64 or t.dim() != 3:
-            raise ValueError("expected a [batch][limbs][N] uint64 tensor")
+    def _check_poly(t: torch.Tensor, limbs: int, n: int, dtype: torch.dtype = torch.uint64) -> None:
+        if t.dtype != dtype or t.dim() != 3:
+            raise ValueError(f"expected a [batch][limbs][N] {str(dtype).removeprefix('torch.')} tensor")
         if t.shape[1] < limbs or t.shape[2] != n or t.stride(2) != 1 or t.stride(1) != n:
             raise ValueError("limb-major [batch][>=limbs][N] layout with contiguous limbs required")
         if t.device.type != "cuda":
@@ -944,7 +944,7 @@ class CKKSContext:
                  out: torch.Tensor | None = None, prime_idx=None, rows: bool = False) -> torch.Tensor:
         """Baby-step partial sums res[c][g][i] = sum_b pts[g*nb + b] * baby_b[i][c] (exact residues).
         babies_c0/c1: one [inputs][>=limbs][N] tensor per baby step (same batch stride); limb l
-        uses prime prime_idx[l] (default: the first ``limbs`` Q primes)."""
+        uses prime prime_idx[l] (default: the first ``limbs`` Q primes).  ``rows``: ``bsgs_mac_rows``."""
 
         prime_idx = self.q_prime_idx(limbs) if prime_idx is None else list(prime_idx)
         if len(prime_idx) != limbs:
@@ -959,16 +959,18 @@ class CKKSContext:
             self._check_poly(t, limbs, self.N)
             if t.shape[0] != ni or _bstride(t) != stride:
                 raise ValueError("baby tensors need one shape and batch stride")
-        self._check_poly(pts, limbs, self.N)
+        fn, name, words = nat.lib().hck_bsgs_mac, "hck_bsgs_mac", torch.uint64
+        if rows:
+            if not self.rows_mac or ni > nat.HCK_MAC_ROWS_INPUTS:
+                raise nat.NativeError(f"hck_bsgs_mac_rows takes at most {nat.HCK_MAC_ROWS_INPUTS} inputs, FP64 words")
+            fn, name, words = nat.lib().hck_bsgs_mac_rows, "hck_bsgs_mac_rows", torch.float64
+        self._check_poly(pts, limbs, self.N, words)
         if pts.shape[0] != giants * nb:
             raise ValueError(f"expected {giants * nb} plaintext rows, got {pts.shape[0]}")
         if out is None:
             out = self.empty(2, giants, ni, limbs, self.N)
         if tuple(out.shape) != (2, giants, ni, limbs, self.N) or not out.is_contiguous():
             raise ValueError("out must be a contiguous [2][giants][inputs][limbs][N] tensor")
-        fn, name = nat.lib().hck_bsgs_mac, "hck_bsgs_mac"
-        if rows:
-            fn, name = nat.lib().hck_bsgs_mac_rows, "hck_bsgs_mac_rows"
         nat.check(fn(self._h, limbs, nat.int_array(prime_idx), ni, nb, giants,
                      nat.ptr_array([t.data_ptr() for t in babies_c0]),
                      nat.ptr_array([t.data_ptr() for t in babies_c1]), stride, pts.data_ptr(), _bstride(pts),
@@ -994,7 +996,7 @@ class CKKSContext:
         return 4 * giants >= 3 * -(-giants // slots) * slots
 
     def bsgs_mac_rows(self, babies_c0, babies_c1, pts: torch.Tensor, limbs: int, giants: int) -> torch.Tensor:
-        """``bsgs_mac`` of at most two inputs with plaintexts from ``encode(...,
+        """``bsgs_mac`` of at most two inputs with the float64 plaintexts of ``encode(...,
         row_pass=False)``: their row pass runs inside the product (hck_bsgs_mac_rows); the same residues
         as encoding them whole."""
 
@@ -1053,8 +1055,8 @@ class CKKSContext:
         ``flags`` tensor ([>= rows] int32, zeroed once) the flags accumulate there for one check
         at the caller's next synchronisation point (``check_encode_flags``).
 
-        ``row_pass=False`` (contexts with ``rows_mac``) stops after the transform's column pass: the
-        words are doubles that only ``bsgs_mac_rows`` reads (hck_encode_cols)."""
+        ``row_pass=False`` (contexts with ``rows_mac``) stops after the transform's column pass
+        (hck_encode_cols): the result is float64, and only ``bsgs_mac_rows`` takes it."""
 
         for v in (values,) + ((values_im,) if values_im is not None else ()):
             if v.dtype != torch.float64 or v.dim() != 2 or v.shape[1] != self.max_slots:
@@ -1070,9 +1072,10 @@ class CKKSContext:
         prime_idx = self.q_prime_idx(limbs) if prime_idx is None else list(prime_idx)
         if len(prime_idx) != int(limbs):
             raise ValueError("one prime index per limb")
+        words = torch.uint64 if row_pass else torch.float64
         if out is None:
-            out = self.empty(rows, limbs, self.N)
-        self._check_poly(out, limbs, self.N)
+            out = torch.empty((rows, limbs, self.N), dtype=words, device=self.device)
+        self._check_poly(out, limbs, self.N, words)
         own = flags is None
         if own:
             flags = torch.zeros(max(rows, 1), dtype=torch.int32, device=self.device)

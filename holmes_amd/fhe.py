@@ -83,11 +83,22 @@ class Plaintext:
         self.cv = []
 
 
-class ColumnPlaintext(Plaintext):
+class ColumnPlaintext:
     """Plaintext rows that have had the transform's column pass only (``CKKSContext.encode(...,
-    row_pass=False)``): ``hoisted_mac_sum`` finishes them inside its multiply-accumulate."""
+    row_pass=False)``): ``rows`` is ``[batch][limbs][N]`` float64, which ``hoisted_mac_sum`` finishes
+    inside its multiply-accumulate.  No ``Plaintext``: there is no NTT-domain polynomial that other
+    operations could read."""
 
-    __slots__ = ()
+    __slots__ = ("rows", "state", "slots")
+
+    def __init__(self, rows: torch.Tensor, state: CipherState, *, slots: int):
+        self.rows = rows
+        self.state = state
+        self.slots = int(slots)
+
+    def __getattr__(self, name):
+        raise AttributeError(f"plaintext rows without the transform's row pass have no {name!r}: "
+                             "only hoisted_mac_sum takes them")
 
 
 def generate_client_context(spec: CKKSContextSpec, device: str = "cuda"):
@@ -613,7 +624,8 @@ def hoisted_mac_sum(ct: Cipher, baby_offsets, plaintexts: Plaintext, giant_offse
                     baby_rotations=None) -> Cipher:
     """One BSGS chunk: sum_g rot(sum_b pt[g B + b] * baby_b, g * giant_offset) for every batch row
     of ``ct`` (llama3fhe/operators/linear/operator.py:434-444).  The baby MAC runs over all rows
-    and giants at once (hck_bsgs_mac).  ``strategy="normal"`` closes the giants by Horner steps
+    and giants at once (hck_bsgs_mac, or hck_bsgs_mac_rows for a ``ColumnPlaintext``).
+    ``strategy="normal"`` closes the giants by Horner steps
     acc <- rot(acc, giant_offset) + partial_g, each one fused rotate-and-add; with
     ``"ext_double_hoist"`` every partial is rotated by its own multiple of giant_offset in the
     extended basis and the sum is closed by one ModDown.  The result keeps the input level with
@@ -631,11 +643,12 @@ def hoisted_mac_sum(ct: Cipher, baby_offsets, plaintexts: Plaintext, giant_offse
     babies = tuple(baby_rotations)
     if len(babies) != nb:
         raise ValueError(f"expected {nb} baby rotations, got {len(babies)}")
-    pts = plaintexts.cv[0] if isinstance(plaintexts, Plaintext) else plaintexts
-    pt_state = plaintexts.state if isinstance(plaintexts, Plaintext) else None
+    columns = isinstance(plaintexts, ColumnPlaintext)
+    pts = plaintexts.rows if columns else plaintexts.cv[0] if isinstance(plaintexts, Plaintext) else plaintexts
+    pt_state = plaintexts.state if isinstance(plaintexts, (Plaintext, ColumnPlaintext)) else None
     if pts.shape[0] != nb * G:
         raise ValueError(f"expected {nb * G} plaintext rows, got {pts.shape[0]}")
-    mac = ctx.bsgs_mac_rows if isinstance(plaintexts, ColumnPlaintext) else ctx.bsgs_mac
+    mac = ctx.bsgs_mac_rows if columns else ctx.bsgs_mac
     part = mac([_view(b.cv[0], limbs) for b in babies], [_view(b.cv[1], limbs) for b in babies],
                pts, limbs, G)  # [2][G][B][limbs][N]
     idx = ctx.q_prime_idx(limbs)

@@ -248,7 +248,8 @@ class LinearWeight:
                   flags: torch.Tensor | None = None, row_pass: bool = True) -> torch.Tensor:
         """Encoded diagonals [giant_count * baby_steps][limbs][N] of ``chunk`` (NTT domain).
         ``flags`` (int32, one per row) defers the overflow check to the caller; ``row_pass=False``
-        leaves the transform's row pass to the multiply-accumulate (``fhe.ColumnPlaintext``)."""
+        leaves the transform's row pass to the multiply-accumulate: float64 words, for a
+        ``fhe.ColumnPlaintext``."""
 
         if self._closed:
             raise RuntimeError("linear weight is closed")

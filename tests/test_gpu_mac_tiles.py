@@ -90,6 +90,23 @@ def test_row_pass_inside_the_product(env, ni, nb, G, limbs):
         ctx.bsgs_mac_rows([ctx.zeros(3, 1, ctx.N)], [ctx.zeros(3, 1, ctx.N)], ctx.zeros(1, 1, ctx.N), 1, 1)
 
 
+def test_rows_without_their_row_pass_are_told_apart(env):
+    """encode(row_pass=False) gives float64: each product refuses the other's plaintexts."""
+    ctx, _ = env
+    if not ctx.rows_mac:
+        return
+    re = torch.randn(4, ctx.max_slots, dtype=torch.float64, device="cuda")
+    whole, cols = ctx.encode(re, 2.0**40, 1), ctx.encode(re, 2.0**40, 1, row_pass=False)
+    assert (whole.dtype, cols.dtype) == (torch.uint64, torch.float64)
+    x = [ctx.zeros(1, 1, ctx.N)]
+    with pytest.raises(ValueError, match="uint64"):
+        ctx.bsgs_mac(x, x, cols, 1, 4)
+    with pytest.raises(ValueError, match="float64"):
+        ctx.bsgs_mac_rows(x, x, whole, 1, 4)
+    with pytest.raises(ValueError, match="float64"):
+        ctx.encode(re, 2.0**40, 1, row_pass=False, out=whole)
+
+
 @pytest.mark.parametrize("D,lanes,shift,B,base,G", [(96, 4, 0, 1, 0, 3), (96, 8, 5, 7, 2, 2), (64, 1, 0, 9, 1, 2),
                                                     (1, 2, 3, 17, 0, 1)])
 def test_packed_baby_chunks(env, D, lanes, shift, B, base, G):
