@@ -983,17 +983,27 @@ class CKKSContext:
 
         return max(self.primes) < 1 << 50
 
-    def rows_mac_pays(self, inputs: int, giants: int) -> bool:
-        """Whether ``bsgs_mac_rows`` beats encoding the plaintexts whole: its kernel takes one or two
-        inputs, 4 or 8 giants a workgroup, and transforms the empty slots' rows too.  Encode and
-        product over 8 babies x 3 limbs up to 32 x 17, times as fast: one input with 4 giants 1.11 to
-        1.47, 6 1.03 to 1.37, 9 1.03 to 1.46, 16 1.17 to 1.52 (1 giant 0.95 to 1.09, 3 0.95 to 1.40); two
-        with 6 1.00 to 1.27, 8 1.08 to 1.39, 16 1.05 to 1.36 (4 0.90 to 1.09, 9 0.91 to 1.15)."""
+    def rows_mac_pays(self, inputs: int, giants: int, limbs: int) -> bool:
+        """Whether ``bsgs_mac_rows`` is at least as fast as encoding the plaintexts whole.  Its kernel
+        takes one or two inputs and 4 or 8 giants a workgroup (the row pass runs for empty slots too), and a
+        workgroup walks the babies of one row one after another: with few limbs and giants there are too
+        few workgroups to hide that.  Encode and product together, times as fast (GPU time, 1 to 32 babies):
+        one input: 1 limb: 4 giants 0.86 to 1.06, 9 0.94 to 1.09, 16 1.00 to 1.06, 32 1.08 to 1.18; 2 limbs: 4 0.97 to
+        1.08, 6 0.93 to 1.08, 8 1.00 to 1.09, 16 1.01 to 1.28; 3 limbs: 4 1.00 to 1.16, 6 1.02 to 1.18; 17 limbs: 4 1.08
+        to 1.45, 6 1.07 to 1.37; three quarters not full: 5 giants 0.88 to 1.08 at 2 limbs, 0.99 to 1.19 at 5.
+        two inputs: 1 limb: 8 0.92 to 1.06, 32 1.06 to 1.12; 2 limbs: 8 0.96 to 1.05, 16 1.01 to 1.21, 20 0.96 to
+        1.07, 24 1.01 to 1.14; 3 limbs: 8 1.03 to 1.21, 12 0.96 to 1.09, 16 1.00 to 1.19; 4 limbs: 7 1.06 to 1.27, 12
+        1.02 to 1.17; 6 limbs: 6 0.95 to 1.14, 7 0.99 to 1.21; 8 limbs: 6 0.97 to 1.25; 17 limbs: 6 1.03 to 1.27, 8
+        1.06 to 1.36; three quarters not full: 9 giants 0.91 to 1.15."""
 
         if not self.rows_mac or not 1 <= inputs <= 2 or giants < 4:
             return False
         slots = 4 if inputs == 1 else 8
-        return 4 * giants >= 3 * -(-giants // slots) * slots
+        if 4 * giants < 3 * -(-giants // slots) * slots:  # less than three quarters of the slots hold a giant
+            return False
+        if inputs == 1:
+            return limbs >= 3 or limbs * giants >= 16
+        return limbs * giants >= 48 or (limbs >= 4 and giants >= 7)
 
     def bsgs_mac_rows(self, babies_c0, babies_c1, pts: torch.Tensor, limbs: int, giants: int) -> torch.Tensor:
         """``bsgs_mac`` of at most two inputs with the float64 plaintexts of ``encode(...,

@@ -368,7 +368,7 @@ class LinearOperator:
         for chunk in chunks:
             args = dict(limbs=limbs, scale=wscale, flags=flags)
             kind = fhe.Plaintext
-            if type(weight) is LinearWeight and ctx.rows_mac_pays(int(x0.shape[0]), int(chunk.giant_count)):
+            if type(weight) is LinearWeight and ctx.rows_mac_pays(int(x0.shape[0]), int(chunk.giant_count), limbs):
                 kind, args["row_pass"] = fhe.ColumnPlaintext, False
             pts = kind(weight.plaintext(plan, chunk, **args), pt_state, slots=xc.slots)
             res = fhe.hoisted_mac_sum(xc, plan.baby_offsets, pts, plan.giant_offset, int(chunk.giant_count), ctx,
