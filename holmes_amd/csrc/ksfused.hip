@@ -1199,7 +1199,7 @@ __device__ __forceinline__ void ipq_finish_rs(double (&ip)[16], double (&x)[16],
   if (acc_limb) {
     load_gal(ad, acc_limb, na, 1u);
 #pragma unroll
-    for (int k = 0; k < 16; ++k) ip[k] += ad[k];  // |.| <= 7.2 p with one of add and acc
+    for (int k = 0; k < 16; ++k) ip[k] += ad[k];  // |.| <= 7.2 p: add and acc never come together (ks_rescaled)
   }
   if (!sub_limb && !twice && scalar == 0.0) {
 #pragma unroll
@@ -1562,6 +1562,7 @@ int ks_rescaled(const hck_context* c, int ell, int batch, const uint64_t* d, lon
   if (c->conv_engine != 1 || ell < 2) return HCK_ERR_UNSUPPORTED;
   if (c->alpha > kSrcMax || c->K > kSrcMax) return HCK_ERR_UNSUPPORTED;
   if (batch < 1 || batch > kMaxBatchF || (acc_b == nullptr) != (acc_a == nullptr)) return HCK_ERR_ARG;
+  if (add && (acc_b || prod_ab)) return HCK_ERR_ARG;  // ipq_finish_rs's sum stays below 8 p with one of them
   const GalF G = gal_uniform(galois);
   const int K = c->K, beta = beta_of(c, ell), ext_l = ell + K, nq = ell - 1;
   const long long n = kN;
