@@ -169,8 +169,9 @@ __global__ __launch_bounds__(kMacThreads) void k_bsgs_mac(uint64_t* __restrict__
 // j + 16 k before the exchange and 16 j + k after it), all babies in turn.  The row's twiddles are the
 // same for every plaintext: stages 8..11 in registers (uniform), 12..15 in LDS.  A baby's ciphertext row is
 // shared by the slots through LDS (two buffers, word 16 j + k at 17 k + j).  The next baby's words are in
-// flight while the current one is transformed.  |v| <= 5.5 p after the transform: |term| <= 2.6 p, the
-// sums are reduced every two babies.
+// flight while the current one is transformed.  |v| <= 5.5 p after the transform (centered words, as the
+// encoder's column pass takes them): |term| <= 2.6 p, the sums are reduced every two babies.
+static_assert(kCentered + 2 * mulv_bound(kFwdOut) < kExact, "two babies on a centered sum");
 // SL: with one input 4 giants, a single wave (4, 8, 9, 16 giants x 32 babies: 0.84, 1.49, 1.82, 2.86 ms, 8
 // slots 1.03, 1.50, 2.07, 2.92, 16 slots 1.45, 1.88, 2.00, 2.84: fewer slots stand empty in the last
 // tile); with two inputs 8, since the two rows' words of a single wave spill (8 and 16 giants 1.73 and 3.37 ms,
@@ -293,10 +294,12 @@ __global__ __launch_bounds__(16 * mr_slots(NI), 2) void k_mac_rows(
 
 // The matrix-core MAC's arithmetic for primes below 2^50 (mac_mx.hpp): canonical words below 2^50 have
 // seven balanced digits (the top one at most 4).  The byte-pair sums a_k (|a_k| < 2^29, a_6 the top
-// digit's own sum, below 2^9) give d0 + 2^32 d1 + 2^64 d2 with |d0|, |d1| < 2^46 and |d2| < 2^46:
-// 2^32 d1 is exact, its quotient rint(2^32 d1 / p) leaves an exact remainder within 0.51 p, and
-// d2 * (2^64 mod p) is one lazy product within 0.51 p.  Four steps of 16 babies stay below
-// 4 (2^46 + 1.1 p) < 2^53, so the running sum is reduced once, in finish().
+// digit's own sum, below 2^9) give d0 + 2^32 d1 + 2^64 d2 with |d0|, |d1| and |d2| < 2^46, taken by
+// Horner's rule: u = d1 + (2^32 d2 mod p), then d0 + (2^32 u mod p).  A product by 2^32 is exact, and the FMA
+// with its rounded quotient leaves the exact remainder, within 0.51 p for p near 2^50 (for small primes
+// the words have fewer digits, the sums are smaller and a quotient off by a few units leaves a few p, far
+// below 2^46).  Four steps of 16 babies stay below 4 (2^46 + 1.1 p) < 2^53, so the running sum is
+// reduced once, in finish().
 struct MxFp {
   static constexpr int ND = 7;
   typedef DevTables Tables;

@@ -73,7 +73,7 @@ __device__ __forceinline__ void gs_bf(double& u, double& v, const double w, doub
 }
 
 // ----------------------------------------------------------------- column transforms (16 threads)
-// forward stages 0..3 on layout A (inputs within p/2 + 1)
+// forward stages 0..3 on layout A (centered inputs)
 __device__ __forceinline__ void col_fwd_lo(double (&x)[16], const double* __restrict__ tw, double p, double pinv) {
 #pragma unroll
   for (int l = 0; l < 4; ++l) {
@@ -484,10 +484,10 @@ __device__ __forceinline__ uint64_t digit_word(double y) {
   return ((uint64_t)__double_as_longlong(t) + (M - 0x4338000000000000ULL)) ^ M;
 }
 
-// sum_c C_c 256^c (+ r) mod p into [-p/2 - 1, p/2 + 1] (|C_c| < 2^20, |r| < 2^49): lo = C_0..C_3 part
+// sum_c C_c 256^c (+ r) mod p into p/2 + 2^12 on either side (|C_c| < 2^20, |r| < 2^49): lo = C_0..C_3 part
 // (|lo| < 2^45) + r, hi = C_4..C_6 part (|hi| < 2^37), value lo + 2^32 hi.  The value is below 2^13 p
-// (56 digits times centered constants), so rint of its estimated quotient leaves it within p/2 + 1;
-// hi 2^32 - q p is then an integer below 2^51 and the FMA exact.  k32 = 2^32 / p.
+// (56 digits times centered constants), so its quotient's estimate is off by 2^-38 at most: 2^12 below
+// 2^50, well inside kCentered.  hi 2^32 - q p is then an integer below 2^51 and the FMA exact.  k32 = 2^32 / p.
 // The pairs a = C_0 + 256 C_1, b = C_2 + 256 C_3, d = C_4 + 256 C_5 and C_6 (each |.| < 2^29).
 __device__ __forceinline__ double mconv_fold_lohi(double lo, double hi, double p, double pinv, double k32) {
   const double q = __builtin_rint(__builtin_fma(hi, k32, lo * pinv));
@@ -861,8 +861,8 @@ __device__ __forceinline__ void rows_fwd_lds(double (&x)[16], double* S, const d
 // tile load is issued as soon as the previous transform has left its result in S, behind that
 // digit's key loads, so the tile lands while the inner product runs.  After the last digit, `after`
 // (a workspace limb, or null) is loaded into x for the caller.  TW must hold the forward twiddles
-// (visible).  With ``zero`` false the products are added to sb / sa (|sb|, |sa| <= p/2 + 1 on entry:
-// the grouped kernel's running sums).  Returns |sb|, |sa| <= p/2 + 1.
+// (visible).  With ``zero`` false the products are added to sb / sa (centered on entry: the grouped
+// kernel's running sums).  Returns centered sums.
 // Hoisted digits (HoistSrc::digits non-null): the extended digits of every input were materialised
 // once in the full NTT domain (natural layout, canonical u64, [input][beta][ell + K] limbs, the own
 // digit's limbs unused), and item b rotates input (src0 + b) mod inputs: each digit is then read
@@ -959,8 +959,8 @@ __device__ __forceinline__ void tile_ip_body(double (&sb)[16], double (&sa)[16],
     }
   }
   if constexpr (HOIST) {
-    // canonical digits read through sigma_g: |term| <= 0.9p; a reduction every three digits keeps
-    // the sums below p/2 + 1 + 0.9p + 3 * 0.9p < 8p <= 2^53
+    // canonical digits read through sigma_g: |term| <= 0.9p, a reduction every three digits
+    static_assert(kCentered + 4 * mulv_bound(1.0) < kExact, "own digit and three more");
     for (int n = 0; n < I.nt2; ++n) {
       const int jd = I.t2digit(n);
       if (n > 0 || OWN_ALWAYS || I.own >= 0 || !pre) {
@@ -998,10 +998,12 @@ __device__ __forceinline__ void tile_ip_body(double (&sb)[16], double (&sa)[16],
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
       const double v = S[s_out(k)];
-      sb[k] += mulv(v, u2d(kb[k]), p, pinv);  // |v| <= 5.5p: |term| <= 2.6p
+      sb[k] += mulv(v, u2d(kb[k]), p, pinv);  // |v| <= kFwdOut p = 5.5p: |term| <= 2.6p
       sa[k] += mulv(v, u2d(ka[k]), p, pinv);
     }
-    if (n % 2 == 1 && n + 1 < I.nt2) {  // <= p/2 + 1 + 2 * 2.6p (+ 0.9p for the own digit) < 8p <= 2^53 between
+    // between reductions the own digit's term and two of a transform, on a centered sum: 6.6p
+    static_assert(kCentered + mulv_bound(1.0) + 2 * mulv_bound(kFwdOut) < kExact, "own digit and two more");
+    if (n % 2 == 1 && n + 1 < I.nt2) {
 #pragma unroll
       for (int k = 0; k < 16; ++k) { sb[k] = reduce(sb[k], p, pinv); sa[k] = reduce(sa[k], p, pinv); }
     }
@@ -1084,7 +1086,8 @@ __device__ __forceinline__ void rows_ip_body(const uint64_t* __restrict__ d, lon
   // ACCP holds tiles / 16 limbs per component from e0 on: the K special limbs, or (ModDown fused
   // with the rescale, e0 = ell - 1) the q_{ell-1} limb first, as Z = P * acc + IP.
   const int k1 = tiles >> 4;
-  if (e < ell && (add || acc_b)) {  // Z = IP + P (sigma(add) + acc): |sb| <= p/2 + 1 + 3 p before the reduction
+  if (e < ell && (add || acc_b)) {  // Z = IP + P (sigma(add) + acc): |sb| <= 2.1 p before the reduction
+    static_assert(kCentered + 2 * mulc_bound(1.0) < kExact, "Z");
     const TwPair pm = T.pmodq[pi];
     double t[16];
     if (add) {
@@ -1146,7 +1149,8 @@ __device__ __forceinline__ void ipq_finish(double (&ip)[16], double (&x)[16], co
   double ad[16];
   if (add_limb) load_gal(ad, add_limb, na, g);
 #pragma unroll
-  for (int k = 0; k < 16; ++k) ip[k] = mulc(ip[k] - S[s_out(k)], pinv_P, p);  // |ip - v| <= 6 p: |r| <= 2.8 p
+  for (int k = 0; k < 16; ++k) ip[k] = mulc(ip[k] - S[s_out(k)], pinv_P, p);  // |ip - v| <= 6 p: |r| <= 2 p
+  static_assert(kCentered + kFwdOut < kExact && mulc_bound(kCentered + kFwdOut) + 2 < kExact, "ModDown finish");
   if (add_limb) {
 #pragma unroll
     for (int k = 0; k < 16; ++k) ip[k] += ad[k];
@@ -1154,7 +1158,7 @@ __device__ __forceinline__ void ipq_finish(double (&ip)[16], double (&x)[16], co
   if (acc_limb) {
     load_gal(ad, acc_limb, na, 1u);
 #pragma unroll
-    for (int k = 0; k < 16; ++k) ip[k] += ad[k];  // |r| <= 4.8 p
+    for (int k = 0; k < 16; ++k) ip[k] += ad[k];  // |r| <= 4 p
   }
 #pragma unroll
   for (int k = 0; k < 16; ++k) o[16 * k] = d2u(canon(ip[k], p, pinv));
@@ -1176,9 +1180,12 @@ __device__ __forceinline__ void ipq_finish_rs(double (&ip)[16], double (&x)[16],
   rows_fwd_lds(x, S, TW, p, pinv);
   if (next) load_t(x, next, rg);
 #pragma unroll
-  for (int k = 0; k < 16; ++k) ip[k] = mulc(ip[k], pinv_P, p) - S[s_out(k)];  // |.| <= 0.7 p + 5.5 p
+  for (int k = 0; k < 16; ++k) ip[k] = mulc(ip[k], pinv_P, p) - S[s_out(k)];  // |.| <= 0.63 p + 5.5 p
+  constexpr double kIp = mulc_bound(kCentered) + kFwdOut;
+  constexpr double kSum = kIp + 2 * mulv_bound(1.0);  // 7.9 p: two tensor products, more than one addend (1 p)
+  static_assert(kSum < kExact && kIp + 1 < kSum, "finish of the fused rescale");
   double ad[16];
-  if (px1) {  // the tensor term formed here: x1 y1 (+ x2 y2), each product within 0.875 p, the sum below 8 p
+  if (px1) {  // the tensor term formed here: x1 y1 (+ x2 y2), each product within 0.875 p
     double t[16];
     load_gal(ad, px1, na, 1u);
     load_gal(t, py1, na, 1u);
@@ -1199,7 +1206,7 @@ __device__ __forceinline__ void ipq_finish_rs(double (&ip)[16], double (&x)[16],
   if (acc_limb) {
     load_gal(ad, acc_limb, na, 1u);
 #pragma unroll
-    for (int k = 0; k < 16; ++k) ip[k] += ad[k];  // |.| <= 7.2 p: add and acc never come together (ks_rescaled)
+    for (int k = 0; k < 16; ++k) ip[k] += ad[k];  // |.| <= 7.1 p: add and acc never come together (ks_rescaled)
   }
   if (!sub_limb && !twice && scalar == 0.0) {
 #pragma unroll
@@ -1208,6 +1215,7 @@ __device__ __forceinline__ void ipq_finish_rs(double (&ip)[16], double (&x)[16],
   }
 #pragma unroll
   for (int k = 0; k < 16; ++k) {  // |r| <= 2.5 p: |2 r - sub + scalar| <= 7 p
+    static_assert(2 * mulc_bound(kSum) + 2 < kExact, "post-ops");
     const double r = mulc(ip[k], ql_inv, p);
     ip[k] = (twice ? 2.0 * r : r) + scalar;
   }
@@ -1336,7 +1344,7 @@ __global__ __launch_bounds__(kT, 2) void k_ks_rows_ip_sum(const uint64_t* __rest
       load_gal(ad, add + (long long)b * add_stride + (long long)e * kN, na, g);
       const TwPair pm = T.pmodq[pi];
 #pragma unroll
-      for (int k = 0; k < 16; ++k) sb[k] = reduce(sb[k] + mulc(ad[k], pm, p), p, pinv);  // back to p/2 + 1
+      for (int k = 0; k < 16; ++k) sb[k] = reduce(sb[k] + mulc(ad[k], pm, p), p, pinv);  // centered again
     }
   }
   if (acc_b) {
@@ -1442,7 +1450,8 @@ __global__ __launch_bounds__(kT) void k_ks_rows_finish(const double* __restrict_
   const TwPair pi_ = inv[i];
   uint64_t* o = out + (long long)pl * out_pstride + (long long)i * kN + na;
 #pragma unroll
-  for (int k = 0; k < 16; ++k) o[16 * k] = d2u(canon(mulc(a[k] - x[k], pi_, p), p, pinv));  // |a - x| <= 6.5 p
+  for (int k = 0; k < 16; ++k) o[16 * k] = d2u(canon(mulc(a[k] - x[k], pi_, p), p, pinv));
+  static_assert(1 + kFwdOut < kExact, "a - x");
 }
 
 // ----------------------------------------------------------------- NTT rows + canonical store
@@ -1843,7 +1852,7 @@ struct LcRsArgs {
 };
 
 // the combination of limb `limb` of group g's terms for row group rg, natural layout (reduced to
-// within p/2 + 1): weights w[t][limb] ([terms][ell]), reduced every 7 terms (|acc| < 8 p)
+// within p/2 + 2): weights w[t][limb] ([terms][ell]), reduced every 7 terms
 __device__ __forceinline__ void lc_tile(double (&acc)[16], const LcRsArgs& A, int g, int terms,
                                         const uint64_t* __restrict__ w, int ell, int limb, long long na, double p,
                                         double pinv) {
@@ -1854,6 +1863,7 @@ __device__ __forceinline__ void lc_tile(double (&acc)[16], const LcRsArgs& A, in
     const double wt = u2d(w[(long long)t * ell + limb]);
 #pragma unroll
     for (int k = 0; k < 16; ++k) acc[k] += mulv(u2d(xl[16 * k]), wt, p, pinv);  // |term| <= 0.875 p
+    static_assert(kCentered + 7 * mulv_bound(1.0) < kExact, "seven terms on a centered sum");
     if (t % 7 == 6) {
 #pragma unroll
       for (int k = 0; k < 16; ++k) acc[k] = reduce(acc[k], p, pinv);
@@ -1893,7 +1903,8 @@ __global__ __launch_bounds__(kT) void k_lc_finish(const LcRsArgs A, int terms, c
   const double ad = ((add_mask >> g) & 1ull) ? u2d(A.add[i]) : 0.0;
   uint64_t* o = A.out[g] + (long long)i * kN + na;
 #pragma unroll
-  for (int k = 0; k < 16; ++k) o[16 * k] = d2u(canon(mulc(a[k] - x[k], qi, p) + ad, p, pinv));  // |a - x| <= 6.5 p
+  for (int k = 0; k < 16; ++k) o[16 * k] = d2u(canon(mulc(a[k] - x[k], qi, p) + ad, p, pinv));
+  static_assert(kCentered + kFwdOut < kExact, "a - x");
 }
 
 size_t lincomb_rescale_bytes(const hck_context* c, int ell, int groups) {

@@ -271,13 +271,14 @@ __global__ __launch_bounds__(kThreads) void k_inv_cols(void* data, long long str
 // * scale, rounded half away from zero: coefficient n < N/2 from the real part of slot brev(n),
 // n >= N/2 from the imaginary part of slot brev(n - N/2)), then for each of its limbs (lpb of them
 // from blockIdx.y lpb: a launch of few rows still fills the chip) takes the centered residue and
-// runs stages 0..7 exactly as k_fwd_cols<kU64> does on stored residues, so the result is
-// bit-identical to rounding, storing every limb and transforming.  The residues of all limbs never
-// reach HBM.  Grid (16, limb chunks, rows).
+// runs stages 0..7.  Its words are congruent to those of k_fwd_cols<kU64> on stored (canonical) residues, so
+// after the row pass, which canonicalises, the result is bit-identical to rounding, storing every limb and
+// transforming.  The residues of all limbs never reach HBM.  Grid (16, limb chunks, rows).
 // Encoder cap: |coefficient| < 2^61, the reference's MAX_ENCODED_BITS
 // (llama3fhe/operators/attention/prefill/softmax.py:559).  A rounded coefficient is an exact double
-// (at and above 2^53 every double is an integer), and reduce() centers it exactly: q = rint(x / p) is
-// below 2^30 and the residue x - q p the exact result of one FMA.
+// (at and above 2^53 every double is an integer), and reduce() centers it exactly: the quotient's estimate
+// is off by |x| / p 2^-52, so the residue x - q p lies within p/2 + 2^9 (kCentered) and is the exact result
+// of one FMA.
 constexpr double kEncodeCap = 2305843009213693952.0;  // 2^61
 
 // One limb's constants.  The tables are read only while the kernel runs: the uniform ones go through
