@@ -181,7 +181,7 @@ constexpr int mr_slots(int inputs) { return inputs == 1 ? 4 : 8; }
 
 template <int NI>
 __global__ __launch_bounds__(16 * mr_slots(NI), 2) void k_mac_rows(
-    uint64_t* __restrict__ res, BabyPtrs babies, long long baby_stride, int nb, int ni, int G,
+    uint64_t* __restrict__ res, BabyPtrs babies, long long baby_stride, int nb, int G,
     const double* __restrict__ pts, long long pt_stride, int limbs, MacPrimes mp, int tiles_g, DevTables T) {
   constexpr int NC = 2 * NI;  // component c of input i: row 2 i + c
   constexpr int SL = mr_slots(NI), TH = 16 * SL, XR = 16 / SL;  // row words per thread and component
@@ -217,10 +217,10 @@ __global__ __launch_bounds__(16 * mr_slots(NI), 2) void k_mac_rows(
     for (int k = 0; k < 16; ++k) d[k] = prow[(long long)b * pt_stride + 16 * k];
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
-      const int i = c >> 1;
+      const long long i = c >> 1;
       const uint64_t* base = (c & 1) ? babies.c1[b] : babies.c0[b];
 #pragma unroll
-      for (int r = 0; r < XR; ++r) xw[c][r] = base[(i < ni ? i : 0) * baby_stride + ln + t + r * TH];
+      for (int r = 0; r < XR; ++r) xw[c][r] = base[i * baby_stride + ln + t + r * TH];
     }
   };
   auto put = [&](int buf) {
@@ -277,14 +277,14 @@ __global__ __launch_bounds__(16 * mr_slots(NI), 2) void k_mac_rows(
 #pragma unroll
     for (int k = 0; k < 16; ++k) v[k] = vn[k];
   }
-  const long long is = (long long)limbs * kN, gs = (long long)ni * is, cs = (long long)G * gs;
+  const long long is = (long long)limbs * kN, gs = NI * is, cs = (long long)G * gs;
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
     const int i = c >> 1;
 #pragma unroll
     for (int k = 0; k < 16; ++k) acc[c][k] = canon(acc[c][k], p, pinv);
     col_b_to_a(acc[c], Rs, j);
-    if (i < ni && tile * SL + s < G) {
+    if (tile * SL + s < G) {
       uint64_t* o = res + (c & 1) * cs + (long long)g * gs + (long long)i * is + ln + j;
 #pragma unroll
       for (int k = 0; k < 16; ++k) o[16 * k] = d2u(acc[c][k]);
@@ -498,7 +498,7 @@ extern "C" int hck_bsgs_mac_rows(const hck_context* ctx, int limbs, const int* p
   if (blocks > 0x7fffffffLL) return HCK_ERR_ARG;
   auto k = inputs == 1 ? hck::k_mac_rows<1> : hck::k_mac_rows<2>;
   k<<<dim3((unsigned)blocks), 16 * slots, 0, (hipStream_t)stream>>>(
-      res, bp, baby_stride, babies, inputs, giants, pts, pt_stride, limbs, mp, tiles_g, ctx->dev);
+      res, bp, baby_stride, babies, giants, pts, pt_stride, limbs, mp, tiles_g, ctx->dev);
   HCK_CHECK_LAUNCH();
   return HCK_OK;
 }
