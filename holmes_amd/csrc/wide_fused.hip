@@ -483,6 +483,7 @@ template <bool INIT = true, bool FINISH = true, bool PIPE = true>
 __device__ __forceinline__ void wtile_ip(u64 (&sb)[16], u64 (&sa)[16], u64 (&x)[16], int& cnt, const WIp& I, int b,
                                          int e, int pi, int rg, uint32_t g, u64* S, const u64* __restrict__ tw,
                                          const u64* __restrict__ tws, const WideTables& T) {
+  static_assert(PIPE || !FINISH, "the sums of a form that is not pipelined are finished by the caller");
   const u64 p = T.p[pi], pi64 = opaque_s(0 - T.mneg[pi]);
   const RowMap mt = map_t(), mn = map_n();
   const int ext_l = I.ell + I.K;
