@@ -97,4 +97,11 @@ __host__ __device__ __forceinline__ uint64_t mulshoup_lazy(uint64_t a, uint64_t 
   return mulshoup_add(a, c, cs, p, 0);
 }
 
+// The same with two 64-bit products: shorter where c is uniform over a wave and nothing is added (an
+// instruction takes one scalar operand, and the chain above pays a move for each further one).
+__host__ __device__ __forceinline__ uint64_t mulshoup_uniform(uint64_t a, uint64_t c, uint64_t cs, uint64_t p) {
+  const uint64_t q = (uint64_t)(((u128_t)a * cs) >> 64);
+  return a * c - q * p;
+}
+
 }  // namespace hck

@@ -815,7 +815,9 @@ __global__ __launch_bounds__(kWMacThreads) void wk_bsgs_mac(const WMac P, long l
 // one Shoup product by 2^60 mod p (below 2p) added to S0; the invariant S0 < 2^30 + 2p, S1 < 2^30,
 // S2 = 0 keeps kSFold more steps inside 64 bits (2^30 + 2^61 + 7 2^60 and 2^30 + 7 2^61 + 2^34 below
 // 2^64).  The result is the canonical residue of S0 + S1 2^30 (below 2^62), the value sum_b x_b w_b
-// mod p exactly, as the 128-bit MAC gives it.  Tiles of kSTI inputs x kSTG giants per thread.
+// mod p exactly, as the 128-bit MAC gives it.  Tiles of kSTI inputs x kSTG giants per thread.  The folds'
+// product by 2^60 as mulshoup_uniform: 2998 VALU instructions in all where mulshoup_lazy gives 3398 (9
+// inputs x 8 babies x 8 giants x 24 limbs 1491 -> 1461 us, 3 x 16 x 16 x 8 585 -> 566 us).
 constexpr int kSTI = 2;
 constexpr int kSTG = 4;
 constexpr int kSFold = 7;
@@ -898,7 +900,7 @@ __global__ __launch_bounds__(kWMacThreads) void wk_bsgs_mac30(const WMac P, long
             a &= kM30;
             h += m >> 30;
             m &= kM30;
-            s0[t][c][g] = a + mulshoup_lazy(h, c60, c60s, p);
+            s0[t][c][g] = a + mulshoup_uniform(h, c60, c60s, p);
             s1[t][c][g] = m;
             s2[t][c][g] = 0;
           }
@@ -936,7 +938,7 @@ __global__ __launch_bounds__(kWMacThreads) void wk_bsgs_mac30(const WMac P, long
           a &= kM30;
           h += m >> 30;
           m &= kM30;
-          const u64 v = a + (m << 30) + mulshoup_lazy(h, c60, c60s, p);  // below 2^61 + 2^30
+          const u64 v = a + (m << 30) + mulshoup_uniform(h, c60, c60s, p);  // below 2^61 + 2^30
           res[c * cs + (long long)(g0 + g) * gs + (long long)(i0 + t) * is + ln] = wfold128((u128)v, p, mneg, r, rs);
         }
   }
