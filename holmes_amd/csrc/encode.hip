@@ -40,32 +40,34 @@ __device__ __forceinline__ void sbf(Cx& u, Cx& v, double wr, double wi) {
   v.im = dr * wi + di * wr;
 }
 
-// Thread: one slot of one giant, kPackBabies baby steps.  Neighbouring baby steps read neighbouring words
-// of a weight row, so a thread's reads share cache lines and its index arithmetic (64-bit remainders) is
-// paid once: 512 diagonals of a 4096 x 4096 weight 133 -> 94 us (one thread per word before).
-constexpr int kPackBabies = 8;
-
+// Thread: one slot of one giant, KB baby steps.  Neighbouring baby steps read neighbouring words of a weight
+// row, so a thread's reads share cache lines and its index arithmetic (64-bit remainders) is paid once: 512
+// diagonals of a 4096 x 4096 weight 133 -> 94 us (one thread per word before).  KB is 8, or the least power
+// of two that holds all baby steps: a thread of 8 reads all of them whatever it keeps, and with a row per
+// giant those words come from 8 times the cache lines (64 rows, lane shift 512, 1 baby step: 8 a thread
+// 42.8 us, 1 a thread 15.4; 2 baby steps 25.4 and 14.9 at 2; 4 16.2 and 12.5 at 4).
+template <int KB>
 __global__ __launch_bounds__(256) void k_pack_diagonals(const double* __restrict__ W, int D, int lanes,
                                                         int lane_shift, int baby_steps, int chunks, int giant_base,
                                                         double* __restrict__ out) {
   const unsigned s = blockIdx.x * 256 + threadIdx.x;
-  const int gr = blockIdx.y / chunks, b0 = (blockIdx.y % chunks) * kPackBabies;
-  const int n = min(kPackBabies, baby_steps - b0);
+  const int gr = blockIdx.y / chunks, b0 = (blockIdx.y % chunks) * KB;
+  const int n = min(KB, baby_steps - b0);
   const long long g = (long long)giant_base + gr;
   const unsigned f = s / (unsigned)lanes, lane = s % (unsigned)lanes;
   long long o = ((long long)f - g * baby_steps) % D;
   if (o < 0) o += D;
   long long in = ((long long)f + b0 + (long long)lane_shift * lane) % D;
   const double* w = W + o * D;
-  double v[kPackBabies];
+  double v[KB];
 #pragma unroll
-  for (int k = 0; k < kPackBabies; ++k) {
+  for (int k = 0; k < KB; ++k) {
     v[k] = w[in];  // past the last baby step: still inside the row
     in = in + 1 == D ? 0 : in + 1;
   }
   double* q = out + ((long long)gr * baby_steps + b0) * kSlots + s;
 #pragma unroll
-  for (int k = 0; k < kPackBabies; ++k)
+  for (int k = 0; k < KB; ++k)
     if (k < n) q[(long long)k * kSlots] = v[k];
 }
 
@@ -204,8 +206,13 @@ extern "C" int hck_pack_diagonals(const hck_context* ctx, const double* weight, 
     return HCK_ERR_ARG;
   const long long rows = (long long)giant_count * baby_steps;
   if (rows > 65535) return HCK_ERR_ARG;
-  const int chunks = (baby_steps + hck::kPackBabies - 1) / hck::kPackBabies;  // giant_count * chunks <= rows
-  hck::k_pack_diagonals<<<dim3(hck::kSlots / 256, (unsigned)(giant_count * chunks)), 256, 0, (hipStream_t)stream>>>(
+  const int kb = baby_steps == 1 ? 1 : baby_steps == 2 ? 2 : baby_steps <= 4 ? 4 : 8;
+  const int chunks = (baby_steps + kb - 1) / kb;  // giant_count * chunks <= rows
+  auto k = kb == 1   ? hck::k_pack_diagonals<1>
+           : kb == 2 ? hck::k_pack_diagonals<2>
+           : kb == 4 ? hck::k_pack_diagonals<4>
+                     : hck::k_pack_diagonals<8>;
+  k<<<dim3(hck::kSlots / 256, (unsigned)(giant_count * chunks)), 256, 0, (hipStream_t)stream>>>(
       weight, dimension, lanes, lane_shift, baby_steps, chunks, giant_base, out);
   HCK_CHECK_LAUNCH();
   return HCK_OK;

@@ -116,3 +116,10 @@ def test_packed_baby_chunks(env, D, lanes, shift, B, base, G):
     got = ctx.pack_diagonals(torch.from_numpy(W).cuda(), lanes=lanes, lane_shift=shift, baby_steps=B,
                              giant_base=base, giant_count=G).cpu().numpy()
     assert np.array_equal(got, O.pack_diagonals(W, lanes, shift, B, base, G, ctx.max_slots))
+
+
+@pytest.mark.parametrize("D,lanes,shift,B,base,G", [(96, 8, 5, 1, 3, 2), (96, 4, 7, 2, 1, 3), (64, 8, 0, 3, 0, 2),
+                                                    (96, 2, 11, 4, 2, 2), (64, 4, 3, 5, 0, 2), (64, 1, 0, 8, 1, 1)])
+def test_packed_baby_groups(env, D, lanes, shift, B, base, G):
+    """The packer's groups of 1, 2, 4 and 8 baby steps a thread, full and one over."""
+    test_packed_baby_chunks(env, D, lanes, shift, B, base, G)
