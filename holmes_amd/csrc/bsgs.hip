@@ -32,11 +32,15 @@ constexpr int kMacThreads = 128;
 constexpr int kTG = 8;  // giants per thread
 constexpr int kMaxBabies = 64;
 
-// Inputs per thread: the tile that computes the fewest padded rows (measured time per row of the tiles of
-// 4, 3 and 2 inputs 1 : 0.95 : 1.07; a single input has a tile of its own).
-inline int mac_tile_inputs(int ni) {
+// Inputs per thread: the tile that computes the fewest rows, each row of the tiles of 3 and 2 inputs charged
+// with the plaintext words that a smaller tile reads again (an equal count goes to the larger tile).  Tiles
+// of 4 against those of 3: 5, 6 and 9 inputs 1.05 to 1.3 times as long; 13 to 15 1.00 to 1.06 with at most 8
+// giants, 0.94 to 1.0 with 16; 11 and 12 0.94 to 1.0.  Against those of 2: 10 inputs 1.06 to 1.13 with at
+// most 4 giants, 0.90 to 1.0 above with at most 16 babies.  A single input has a tile of its own.
+inline int mac_tile_inputs(int ni, int giants) {
   if (ni == 1) return 1;
-  const int c4 = (ni + 3) / 4 * 4 * 100, c3 = (ni + 2) / 3 * 3 * 95, c2 = (ni + 1) / 2 * 2 * 107;
+  const int w3 = giants <= 8 ? 105 : 107, w2 = giants <= 4 ? 113 : 125;
+  const int c4 = (ni + 3) / 4 * 4 * 100, c3 = (ni + 2) / 3 * 3 * w3, c2 = (ni + 1) / 2 * 2 * w2;
   return c4 <= c3 && c4 <= c2 ? 4 : c3 <= c2 ? 3 : 2;
 }
 
@@ -460,7 +464,7 @@ extern "C" int hck_bsgs_mac(const hck_context* ctx, int limbs, const int* prime_
   }
   const int units_per_limb = hck::kN / hck::kMacThreads;
   const int total_units = limbs * units_per_limb;
-  const int ti = hck::mac_tile_inputs(inputs);
+  const int ti = hck::mac_tile_inputs(inputs, giants);
   const int tiles_i = (inputs + ti - 1) / ti, tiles_g = (giants + hck::kTG - 1) / hck::kTG;
   const int tiles = tiles_i * tiles_g;
   const long long units_padded = ((long long)total_units + hck::kXcds - 1) / hck::kXcds * hck::kXcds;

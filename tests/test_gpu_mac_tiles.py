@@ -58,6 +58,12 @@ def test_vector_tiles(env, ni, nb, G, limbs):
     _check(env, ni, nb, G, limbs)
 
 
+@pytest.mark.parametrize("ni,nb,G,limbs", [(10, 3, 9, 1), (10, 5, 4, 1), (11, 3, 5, 1), (12, 2, 8, 1), (14, 2, 3, 1)])
+def test_vector_tiles_of_many_inputs(env, ni, nb, G, limbs):
+    """More than two input tiles: of 2 or 4 by the giants, of 4 full and one short, of 3."""
+    _check(env, ni, nb, G, limbs)
+
+
 def test_rows_that_are_not_16_byte_aligned(env):
     """A shape of the matrix-core kernel whose plaintexts start at an odd word."""
     _check(env, 8, 16, 16, 1, offset=1)
