@@ -44,6 +44,23 @@ inline int mac_tile_inputs(int ni, int giants) {
   return c4 <= c3 && c4 <= c2 ? 4 : c3 <= c2 ? 3 : 2;
 }
 
+// Where the matrix cores pay on FP64 words: where the tiles are full (mx_pays), and the VALU kernel's own
+// tiles, which need not be, would compute at least `need` of what they compute.  A walk over several tiles keeps
+// one row group per step: it pays earlier than a single tile, which loads both.  Measured, VALU time over
+// matrix-core time at 2 to 20 limbs, (inputs, babies, giants): single tile (8, 11, 16) 0.90 to 0.97, (8, 12, 16)
+// 0.94 to 1.01, (7, 13, 16) 0.94 to 1.05, (8, 14, 16) 1.00 to 1.08, (8, 16, 16) 1.00 to 1.14; two tiles (16, 10,
+// 16) 0.97 to 1.00, (8, 11, 32) 1.02 to 1.07, (16, 12, 16) 1.08 to 1.11; four (16, 10, 32) 1.06 to 1.09, (5,
+// 16, 32) 1.10 to 1.15, (10, 16, 32) 1.13 to 1.19; two steps of babies (8, 20, 16) 0.94 to 1.03, (16, 20,
+// 32) 0.96 to 1.00, (8, 24, 16) 1.08 to 1.15, (16, 33, 16) 1.05 to 1.07.
+inline bool mx_pays_fp(int ni, int nb, int giants) {
+  if (!mx_pays(ni, nb, giants)) return false;
+  auto up = [](int v, int m) { return (v + m - 1) / m * m; };
+  const int tiles = (giants + 15) / 16 * ((2 * ni + 15) / 16);
+  const double need = nb > 16 ? 0.68 : tiles == 1 ? 0.86 : tiles < 4 ? 0.68 : 0.62;
+  const double valu = (double)up(ni, mac_tile_inputs(ni, giants)) * up(giants, kTG) * nb;
+  return valu >= need * up(ni, 8) * up(giants, 16) * up(nb, 16);
+}
+
 struct BabyPtrs {
   const uint64_t* c0[kMaxBabies];
   const uint64_t* c1[kMaxBabies];
@@ -454,7 +471,7 @@ extern "C" int hck_bsgs_mac(const hck_context* ctx, int limbs, const int* prime_
     bp.c0[b] = baby_c0[b];
     bp.c1[b] = baby_c1[b];
   }
-  if (hck::mx_pays(inputs, babies, giants)) {
+  if (hck::mx_pays_fp(inputs, babies, giants)) {
     hck::MxArgs A = hck::mx_args(limbs, mp.prime, inputs, babies, giants, baby_c0, baby_c1, baby_stride, pts, pt_stride, res);
     if (hck::mx_aligned(A)) {
       hck::mx_launch<hck::MxFp>(A, ctx->dev, (hipStream_t)stream);

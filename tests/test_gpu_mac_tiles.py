@@ -58,6 +58,16 @@ def test_vector_tiles(env, ni, nb, G, limbs):
     _check(env, ni, nb, G, limbs)
 
 
+@pytest.mark.parametrize("ni,nb,G,limbs", [(16, 16, 25, 1), (13, 16, 16, 2), (12, 16, 32, 1), (16, 36, 16, 1),
+                                           (16, 40, 31, 1), (8, 14, 16, 3)])
+def test_matrix_core_tiles_with_partial_tiles(env, ni, nb, G, limbs):
+    """Shapes that both widths' rules send to the matrix-core kernel (three quarters of the tiles' volume
+    real) whose last tile of giants, of columns or step of babies is partly empty."""
+    up = lambda v: -(-v // 16) * 16  # noqa: E731
+    assert 4 * G * 2 * ni * nb >= 3 * up(G) * up(2 * ni) * up(nb)
+    _check(env, ni, nb, G, limbs)
+
+
 @pytest.mark.parametrize("ni,nb,G,limbs", [(10, 3, 9, 1), (10, 5, 4, 1), (11, 3, 5, 1), (12, 2, 8, 1), (14, 2, 3, 1)])
 def test_vector_tiles_of_many_inputs(env, ni, nb, G, limbs):
     """More than two input tiles: of 2 or 4 by the giants, of 4 full and one short, of 3."""
