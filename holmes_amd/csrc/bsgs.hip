@@ -6,8 +6,9 @@
 // method that the giant steps then rotate and add (exact-residue semantics of
 // bench/cmp/kernels/holmes_mac.cu:8-12, multi-input tiling of holmes_mac.cu:108-190).
 //
-// Two kernels: with enough inputs, giants and babies to fill its 16 x 16 x 16 tiles the matrix-core MAC
-// of mac_mx.hpp, else k_bsgs_mac on the VALU.  In the latter a thread owns one coefficient of one limb and
+// Three kernels: with enough inputs, giants and babies to fill its 16 x 16 x 16 tiles the matrix-core MAC
+// of mac_mx.hpp, else k_bsgs_mac on the VALU; k_mac_rows for plaintexts that lack the transform's row pass
+// (hck_bsgs_mac_rows).  In k_bsgs_mac a thread owns one coefficient of one limb and
 // a TI x 8 tile of (input, giant) accumulators for both components: per baby step it reads 8 plaintext
 // words and 2 TI baby words for 16 TI products (the next step's words are loaded while the current step
 // computes), so plaintexts stream once per input tile and babies once per giant tile.  Up to 3 inputs HBM

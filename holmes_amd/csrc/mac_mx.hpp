@@ -9,8 +9,8 @@
 // For 16 giants x 16 columns x 16 babies, C_c is two v_mfma_i32_16x16x64_i8 (K = 16 babies x 4 digit
 // bytes): Q_c times the low halves of the columns' digit words plus Q_{c-4} times their high halves,
 // where Q_k holds the plaintext digits w_k, w_{k-1}, w_{k-2}, w_{k-3} of every baby, one byte permute per
-// word.  Each Q_k serves both, and those without a digit in range are left out: 2 ND + 5 products
-// instead of 4 ND - 2.  |C_c| <= 16 babies * ND * 2^14 <= 2^21, exact in int32.  The 2 ND - 1 sums of one
+// word.  Each Q_k serves both, and those without a digit in range are left out: 3 ND - 2 products
+// (19 and 22) instead of 4 ND - 2.  |C_c| <= 16 babies * ND * 2^14 <= 2^21, exact in int32.  The 2 ND - 1 sums of one
 // output are folded into its residue once per 16 babies.
 //
 // What bounds it: one output costs a fold of about 35 (FP64) or 110 (64-bit) VALU instructions per 16
@@ -248,10 +248,23 @@ __global__ __launch_bounds__(kMxThreads, 2) void k_mac_mx(const MxArgs A, const 
 }
 
 // Where the matrix cores pay: by the share of the 16 x 16 x 16 tiles that holds real giants, columns and
-// babies.  Measured at 8 limbs, FP64 words, VALU kernel against this one: share 1: 3.24 / 2.18 ms (16 inputs,
-// 16 babies, 32 giants), 1.66 / 1.15 ms (8, 64, 16); 0.75: 2.50 / 2.00 ms (16, 16, 24), 2.38 / 1.95 ms
-// (16, 24, 16); 0.625: 2.21 / 1.92 ms (10, 16, 32), 1.23 / 1.07 ms (5, 16, 32); 0.5: 1.05 / 1.06 ms (16, 8,
-// 16), 0.93 / 1.00 ms (16, 16, 8), 0.97 / 1.02 ms (4, 16, 32).
+// babies (FP64 words: mx_pays_fp asks for more).  Measured at 8 limbs, VALU kernel against this one, (inputs,
+// babies, giants):
+//   share   FP64 words                          64-bit words
+//   1       3.23 / 2.26 ms (16, 16, 32)         4.72 / 2.70 ms
+//           2.99 / 2.40    (8, 64, 16)          4.05 / 2.74
+//   0.875   1.59 / 1.22    (7, 16, 32)          2.29 / 1.43
+//   0.75    2.39 / 2.09    (16, 16, 24)         3.53 / 2.50
+//           2.28 / 2.02    (16, 24, 16)         3.18 / 2.53
+//   0.625   2.27 / 1.99    (10, 16, 32)         2.91 / 2.49
+//           1.26 / 1.12    (5, 16, 32)          1.75 / 1.36
+//           1.53 / 1.12    (16, 16, 10)         1.73 / 1.35
+//   0.5     1.00 / 1.12    (16, 8, 16)          1.63 / 1.36
+//           0.91 / 1.09    (16, 16, 8)          1.29 / 1.31
+//           0.92 / 1.10    (4, 16, 32)          1.29 / 1.34
+//   0.44    0.95 / 1.07    (7, 8, 32)           1.53 / 1.32
+//   0.375   0.79 / 1.04    (3, 16, 32)          1.21 / 1.28
+// (With 8 babies the 64-bit VALU kernel is slow enough that this one wins below the line too.)
 inline bool mx_pays(int ni, int nb, int G) {
   auto up = [](int v) { return (v + 15) / 16 * 16; };
   return (double)G * (2 * ni) * nb >= 0.6 * up(G) * up(2 * ni) * up(nb);

@@ -9,8 +9,9 @@
 //    (Harvey) butterflies take and return words below 2p; products by twiddles and conversion factors
 //    use Shoup's companions, whose lazy result lies below 2p for any 64-bit input.  Workspace words
 //    keep these lazy ranges;
-//  * key products are Montgomery products x k 2^-64 (below 1.5p for x < 8p, k < p), summed lazily
-//    below 2p and multiplied by 2^64 mod p (Shoup, canonical result) once per output;
+//  * key products are signed Montgomery products x k 2^-64 (wmont_s: in (-p, p / 2) for x < 8p, k < p),
+//    four at a time on sums in [0, 4p) without a reduction, so in (-4p, 6p), and multiplied by 2^64 mod p
+//    (Shoup, canonical result) once per output;
 //  * the base-conversion sums run on the int8 matrix cores with the wide digit tables (wide_dev.hpp:
 //    wdigits takes a canonical residue, wfold returns one).
 // Outputs are canonical.
